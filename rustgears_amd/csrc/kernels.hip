@@ -59,6 +59,7 @@ __global__ void load_probe_kernel() {}
 void load_code_object(hipStream_t s) {
   hipLaunchKernelGGL(load_probe_kernel, dim3(1), dim3(64), 0, s);
   load_requant_code_object(s);
+  load_mid_code_object(s);
 }
 
 // Reads n 16-byte words so that the memory-side cache (256 MB on MI355X)
@@ -1110,15 +1111,12 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64, OCC) void gemm_big_kernel(
   }
 }
 
-// Split-K epilogue: the S partial sums added in slice order, then the fused
-// epilogue (INT8: exact i32 sum; FP16: f32 sum).
+// Split-K epilogue (FP16 and FP32): the S partial f32 sums added in slice
+// order, then the fused epilogue.
 template <int ACT, int MODE>
 __global__ __launch_bounds__(256) void splitk_epilogue_kernel(const int32_t* __restrict__ ws, int S, int64_t M,
                                                               int64_t N, int64_t Mpad, int64_t Npad, Epilogue ep) {
   const int64_t n4 = Npad / 4, total = M * n4;
-  uint32_t amax = 0;
-  float cs = 1.0f;
-  if constexpr (MODE == kModeI8) cs = tensor_scale(ep.absmax_in) * ep.w_scale;
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
     const int64_t row = e / n4, c0 = (e - row * n4) * 4;
     const v4f bias = *reinterpret_cast<const v4f*>(ep.bias + c0);  // padded to Npad
@@ -1126,7 +1124,6 @@ __global__ __launch_bounds__(256) void splitk_epilogue_kernel(const int32_t* __r
     // (a load-add loop waits for each in turn), then added in slice order;
     // past S a lane re-reads the last partial and does not add it.
     constexpr int KB = 8;
-    v4i sum = v4i{0, 0, 0, 0};
     v4f f = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     for (int sp0 = 0; sp0 < S; sp0 += KB) {
       v4i part[KB];
@@ -1138,31 +1135,18 @@ __global__ __launch_bounds__(256) void splitk_epilogue_kernel(const int32_t* __r
 #pragma unroll
       for (int u = 0; u < KB; u++) {
         const bool ok = sp0 + u < S;  // a select, not a branch, so no load waits alone
-        if constexpr (MODE != kModeI8) {
-          const v4f g = f + __builtin_bit_cast(v4f, part[u]);
-          f = ok ? g : f;
-        } else {
-          const v4i g = sum + part[u];
-          sum = ok ? g : sum;
-        }
+        const v4f g = f + __builtin_bit_cast(v4f, part[u]);
+        f = ok ? g : f;
       }
     }
-    if constexpr (MODE != kModeI8) sum = __builtin_bit_cast(v4i, f);
+    const v4i sum = __builtin_bit_cast(v4i, f);
 #pragma unroll
     for (int q = 0; q < 4; q++) {
       const int64_t col = c0 + q;
       if (col < N) {
-        const float v = epi_word<ACT, MODE>(sum[q], cs, bias[q], ep.act_param);
-        ep.y[row * N + col] = v;
-        if (ep.acc_out) ep.acc_out[row * N + col] = sum[q];
-        const uint32_t k = rgmath::absmax_key(v);
-        amax = k > amax ? k : amax;
+        ep.y[row * N + col] = epi_word<ACT, MODE>(sum[q], 1.0f, bias[q], ep.act_param);
       }
     }
-  }
-  if (ep.absmax_out) {
-    amax = wave_max_u32(amax);
-    if ((threadIdx.x & 63) == 0) spread_max(ep.absmax_out, amax);
   }
 }
 
@@ -1227,17 +1211,21 @@ static void launch_gemm_t(const int8_t* A, const int8_t* B, int64_t M, int64_t N
     launch_big<256, 256, 2, 4, 4, 1, 8, MODE>(A, B, M, N, Mpad, Npad, Kpad, ep, 1, nullptr, s);
   } else if (g.kind == 1) {
     launch_big<256, 128, 2, 2, 3, 2, 8, MODE>(A, B, M, N, Mpad, Npad, Kpad, ep, 1, nullptr, s);
-  } else if (g.splits > 1 && ws && ws_bytes >= (int64_t)g.splits * Mpad * Npad * 4) {
-    launch_big<128, 128, 2, 2, 4, 2, 4, MODE>(A, B, M, N, Mpad, Npad, Kpad, ep, g.splits, ws, s);
-    launch_splitk_epilogue<MODE>(ws, g.splits, M, N, Mpad, Npad, ep, s);
   } else {
+    if constexpr (MODE != kModeI8) {
+      if (g.splits > 1 && ws && ws_bytes >= (int64_t)g.splits * Mpad * Npad * 4) {
+        launch_big<128, 128, 2, 2, 4, 2, 4, MODE>(A, B, M, N, Mpad, Npad, Kpad, ep, g.splits, ws, s);
+        launch_splitk_epilogue<MODE>(ws, g.splits, M, N, Mpad, Npad, ep, s);
+        return;
+      }
+    }
     launch_big<128, 128, 2, 2, 4, 2, 4, MODE>(A, B, M, N, Mpad, Npad, Kpad, ep, 1, nullptr, s);
   }
 }
 
 void launch_gemm(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t Mpad, int64_t Npad, int64_t Kpad,
-                 const Epilogue& ep, int32_t* ws, int64_t ws_bytes, hipStream_t s) {
-  launch_gemm_t<kModeI8>(A, B, M, N, Mpad, Npad, Kpad, ep, ws, ws_bytes, s);
+                 const Epilogue& ep, hipStream_t s) {
+  launch_gemm_t<kModeI8>(A, B, M, N, Mpad, Npad, Kpad, ep, nullptr, 0, s);
 }
 
 void launch_gemm_f32(const float* A, const float* B, int64_t M, int64_t N, int64_t Mpad, int64_t Npad,
@@ -1884,28 +1872,24 @@ static void launch_gemv_mfma(const int8_t* A, const int8_t* B, int64_t M, int64_
 // 1024 -> 10, C's 256 -> 10, Q's 32 -> 3).  A 128 x 128 MFMA tile would waste
 // most of its columns, so a wave takes one row at a time instead: lane l
 // holds 16 bytes of every 1 KiB K chunk of the row and of the N weight rows
-// (those are a few KiB and stay in L1), sums them (INT8: sdot4, exact; FP16:
-// fdot2, FP32: FMA, in gemv_kernel's order), and the wave's N sums are
-// reduce-scattered as in gemv_kernel before the fused epilogue.  Kpad is in
-// bytes.  With XQ (INT8) A is the f32 input [M, xk] (xk % 4 == 0, 16-byte
+// (those are a few KiB and stay in L1), sums them (sdot4, exact), and the
+// wave's N sums are reduce-scattered as in gemv_kernel before the fused
+// epilogue.  (FP16 and FP32 heads run in the small-tile GEMM of mid.hip.)
+// With XQ A is the f32 input [M, xk] (xk % 4 == 0, 16-byte
 // aligned rows), quantized as it is read (QuantTensor::from_f32 with the
 // spread slot's scale, quantize.rs:18-24): each value is read once, so the
 // separate quantize pass over it is gone; q_out (capture) receives the i8
 // operand [M, Kpad] and scale_out the scale.
-template <int NN, int MODE, bool XQ = false>
+template <int NN, bool XQ>
 __global__ __launch_bounds__(256) void gemm_narrow_kernel(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
                                                           int64_t M, int64_t N, int64_t Kpad, Epilogue ep, int64_t xk,
                                                           int8_t* q_out, float* scale_out) {
   constexpr int S = pow2_at_least(NN);
   constexpr int SPREAD = 64 / S;
   const int lane = threadIdx.x & 63;
-  float cs = 1.0f, inv = 0.0f;
-  if constexpr (MODE == kModeI8) {
-    const float sa = tensor_scale(ep.absmax_in);
-    cs = sa * ep.w_scale;
-    inv = 1.0f / sa;
-    if (XQ && scale_out && blockIdx.x == 0 && threadIdx.x == 0) *scale_out = sa;
-  }
+  const float sa = tensor_scale(ep.absmax_in);
+  const float cs = sa * ep.w_scale, inv = 1.0f / sa;
+  if (XQ && scale_out && blockIdx.x == 0 && threadIdx.x == 0) *scale_out = sa;
   const int sidx = lane / SPREAD;
   const bool owner = (lane % SPREAD) == 0 && sidx < N;
   const float bias_v = ep.bias[sidx < N ? sidx : N - 1];
@@ -1945,38 +1929,16 @@ __global__ __launch_bounds__(256) void gemm_narrow_kernel(const int8_t* __restri
       for (int n = 0; n < NN; n++) {
         const v4i w = *reinterpret_cast<const v4i*>(B + (int64_t)n * Kpad + kk);
         int32_t c = acc[n];
-        if constexpr (MODE == kModeF32) {
-          const v4f xf = __builtin_bit_cast(v4f, av), wf = __builtin_bit_cast(v4f, w);
-          float f = __int_as_float(c);
-#pragma unroll
-          for (int q = 0; q < 4; q++) f = __builtin_fmaf(xf[q], wf[q], f);
-          c = __float_as_int(f);
-        } else if constexpr (MODE == kModeF16) {
-          const v8h xh = __builtin_bit_cast(v8h, av), wh = __builtin_bit_cast(v8h, w);
-          float f = __int_as_float(c);
-#pragma unroll
-          for (int q = 0; q < 4; q++)
-            f = __builtin_amdgcn_fdot2(v2h{xh[2 * q], xh[2 * q + 1]}, v2h{wh[2 * q], wh[2 * q + 1]}, f, false);
-          c = __float_as_int(f);
-        } else {
-          c = __builtin_amdgcn_sdot4(av[0], w[0], c, false);
-          c = __builtin_amdgcn_sdot4(av[1], w[1], c, false);
-          c = __builtin_amdgcn_sdot4(av[2], w[2], c, false);
-          c = __builtin_amdgcn_sdot4(av[3], w[3], c, false);
-        }
+        c = __builtin_amdgcn_sdot4(av[0], w[0], c, false);
+        c = __builtin_amdgcn_sdot4(av[1], w[1], c, false);
+        c = __builtin_amdgcn_sdot4(av[2], w[2], c, false);
+        c = __builtin_amdgcn_sdot4(av[3], w[3], c, false);
         acc[n] = c;
       }
     }
-    const int32_t mine = wave_reduce_scatter<S, MODE != kModeI8>(acc, lane);
-    float pre;
-    if constexpr (MODE == kModeF16) {
-      pre = rgmath::round_fp16(__int_as_float(mine) + bias_v);
-    } else if constexpr (MODE == kModeF32) {
-      pre = __int_as_float(mine) + bias_v;
-    } else {
-      const float prod = (float)mine * cs;
-      pre = prod + bias_v;
-    }
+    const int32_t mine = wave_reduce_scatter<S, false>(acc, lane);
+    const float prod = (float)mine * cs;
+    const float pre = prod + bias_v;
     if (owner) {
       float v;
       switch (ep.act) {
@@ -2000,7 +1962,7 @@ __global__ __launch_bounds__(256) void gemm_narrow_kernel(const int8_t* __restri
   }
 }
 
-template <int MODE, bool XQ = false>
+template <bool XQ>
 static void launch_gemm_narrow_t(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t Kpad_bytes,
                                  const Epilogue& ep, hipStream_t s, int64_t xk = 0, int8_t* q_out = nullptr,
                                  float* scale_out = nullptr) {
@@ -2009,22 +1971,22 @@ static void launch_gemm_narrow_t(const int8_t* A, const int8_t* B, int64_t M, in
   if (M <= 0) return;
   const int64_t blocks = std::min<int64_t>((M + 3) / 4, 8192);
   if (N <= 4)
-    RG_LAUNCH((gemm_narrow_kernel<4, MODE, XQ>), dim3((unsigned)blocks), dim3(256), 0, s, A, B, M, N, Kpad_bytes, ep,
+    RG_LAUNCH((gemm_narrow_kernel<4, XQ>), dim3((unsigned)blocks), dim3(256), 0, s, A, B, M, N, Kpad_bytes, ep,
               xk, q_out, scale_out);
   else if (N <= 8)
-    RG_LAUNCH((gemm_narrow_kernel<8, MODE, XQ>), dim3((unsigned)blocks), dim3(256), 0, s, A, B, M, N, Kpad_bytes, ep,
+    RG_LAUNCH((gemm_narrow_kernel<8, XQ>), dim3((unsigned)blocks), dim3(256), 0, s, A, B, M, N, Kpad_bytes, ep,
               xk, q_out, scale_out);
   else if (N <= 12)  // the 10-class heads: 12 weight rows per lane instead of 16
-    RG_LAUNCH((gemm_narrow_kernel<12, MODE, XQ>), dim3((unsigned)blocks), dim3(256), 0, s, A, B, M, N, Kpad_bytes,
+    RG_LAUNCH((gemm_narrow_kernel<12, XQ>), dim3((unsigned)blocks), dim3(256), 0, s, A, B, M, N, Kpad_bytes,
               ep, xk, q_out, scale_out);
   else
-    RG_LAUNCH((gemm_narrow_kernel<16, MODE, XQ>), dim3((unsigned)blocks), dim3(256), 0, s, A, B, M, N, Kpad_bytes, ep,
+    RG_LAUNCH((gemm_narrow_kernel<16, XQ>), dim3((unsigned)blocks), dim3(256), 0, s, A, B, M, N, Kpad_bytes, ep,
               xk, q_out, scale_out);
 }
 
 void launch_gemm_narrow(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t Kpad, const Epilogue& ep,
                         hipStream_t s) {
-  launch_gemm_narrow_t<kModeI8>(A, B, M, N, Kpad, ep, s);
+  launch_gemm_narrow_t<false>(A, B, M, N, Kpad, ep, s);
 }
 
 bool gemm_narrow_xq_supported(int64_t K, int64_t Kpad) { return K > 0 && K % 4 == 0 && K <= Kpad && Kpad % 16 == 0; }
@@ -2033,7 +1995,7 @@ void launch_gemm_narrow_xq(const float* x, const int8_t* B, int64_t M, int64_t N
                            const Epilogue& ep, int8_t* q_out, float* scale_out, hipStream_t s) {
   if (!gemm_narrow_xq_supported(K, Kpad) || (reinterpret_cast<uintptr_t>(x) & 15) || !ep.absmax_in)
     throw std::logic_error("narrow GEMM: the quantizing form needs K % 4 == 0, an aligned input and a slot");
-  launch_gemm_narrow_t<kModeI8, true>(reinterpret_cast<const int8_t*>(x), B, M, N, Kpad, ep, s, K, q_out, scale_out);
+  launch_gemm_narrow_t<true>(reinterpret_cast<const int8_t*>(x), B, M, N, Kpad, ep, s, K, q_out, scale_out);
 }
 
 // ---------------------------------------------------------------------------
@@ -2311,6 +2273,15 @@ bool gemm_xq_small_supported(int64_t M, int64_t N, int64_t Npad, int64_t K, int6
   return (int64_t)g.tiles_m * g.tiles_n <= xqs::kMaxBlocks;
 }
 
+// The geometry's time in us: a launch and 35 us per MB that the busiest CU
+// loads (measured: 131 KB 6.4 us, 65 KB 4.4 us, 917 KB 35 us), and the
+// slices' atomic round trip.
+double gemm_xq_small_us(int64_t M, int64_t Npad, int64_t Kpad) {
+  const XqsGeom g = xqs_geom(M, Npad, Kpad);
+  const int64_t wgs = (int64_t)g.tiles_m * g.tiles_n * g.S, per_cu = (wgs + xqs::kTargetGrid - 1) / xqs::kTargetGrid;
+  return 2.0 + 35e-6 * (double)per_cu * g.ks * 64.0 * (xqs::kTM * 4 + g.TN) + (g.S > 1 ? 0.3 : 0.0);
+}
+
 int64_t gemm_xq_small_sync_words(int64_t M, int64_t Npad, int64_t Kpad) {
   const XqsGeom g = xqs_geom(M, Npad, Kpad);
   return g.S > 1 ? (int64_t)g.tiles_m * g.tiles_n * xqs::kTM * g.TN * 2 : 0;
@@ -2552,18 +2523,6 @@ void launch_mlp_tiny(const float* x, float* y, const TinyChain& ch, SlotClear cl
   if (!ok || wbytes > kTinyWeightBytes || (reinterpret_cast<uintptr_t>(x) & 3) || (reinterpret_cast<uintptr_t>(y) & 3))
     throw std::logic_error("mlp_tiny: the chain does not fit the one-workgroup kernel");
   RG_LAUNCH(mlp_tiny_kernel, dim3(1), dim3(tiny::kThreads), 0, s, x, y, ch, clear);
-}
-
-void launch_gemm_narrow_f16(const uint16_t* A, const uint16_t* B, int64_t M, int64_t N, int64_t Kpad_h,
-                            const Epilogue& ep, hipStream_t s) {
-  launch_gemm_narrow_t<kModeF16>(reinterpret_cast<const int8_t*>(A), reinterpret_cast<const int8_t*>(B), M, N,
-                                 2 * Kpad_h, ep, s);
-}
-
-void launch_gemm_narrow_f32(const float* A, const float* B, int64_t M, int64_t N, int64_t Kpad_f, const Epilogue& ep,
-                            hipStream_t s) {
-  launch_gemm_narrow_t<kModeF32>(reinterpret_cast<const int8_t*>(A), reinterpret_cast<const int8_t*>(B), M, N,
-                                 4 * Kpad_f, ep, s);
 }
 
 void launch_gemv(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t Npad, int64_t Kpad,

@@ -147,6 +147,11 @@ struct OpPlan {
   // kernel's barrier words in the slot set, or -1 for the absmax + quantize
   // kernel pair.
   int64_t iq_sync_base = -1;
+  bool mid = false;  // Linear on the small-tile GEMM of mid.hip
+  // FP32 Linear -> Act: the Linear's epilogue applies the activation
+  // (fused_act on it; act_fused on the Act op, which launches nothing).
+  int fused_act = -1;  // the Act op's index
+  bool act_fused = false;
   // FP16 Linear -> FP16 Linear: the producer's GEMM epilogue writes the
   // consumer's binary16 operand (q_ready / q_in of the consumer as above).
   bool handoff = false;
@@ -716,6 +721,35 @@ static int conv_pool_fusion(const rgnpu_program* P, const std::vector<OpPlan>& p
   return conv_pool_supported(c, r16) ? r16 : 0;
 }
 
+// Whether a Linear runs on the small-tile GEMM (mid.hip) rather than the
+// 128 x 128 and larger tiles of launch_gemm: below 128 real tiles of
+// 128 x 128 those leave CUs idle or split K (1000 x 1024 x 1024 i8: 17.6
+// against 5.8 us; above, the larger tiles load less: 1000 x 4096 x 4096 i8
+// 24.9 against 29.5 us, f16 44.4 against 51.2 us).  Exceptions:
+//  * INT8 from 48 tiles on, K not split (up to 7 K steps of 64): the tile GEMM
+//    also quantizes its outputs for the next Linear, and one kernel of it
+//    takes what this one and the quantize pass take (2048 x 384 x 512: 8.6
+//    against 4.8 + 3.7 us).
+//  * INT8 heads of at most 16 outputs quantize as they read (launch_gemm_narrow).
+//  * FP32 is bound by the matrix cores (mid_f32_better).
+// RGNPU_MID=0 turns it off, 2 takes it for every Linear (tests, measurements).
+static bool use_mid(const rgnpu_program* P, const Op& op, const OpPlan& pl) {
+  if (op.kind != OP_LINEAR || op.diag || pl.gemv || pl.rows <= 0) return false;
+  const int64_t es = P->precision == RGNPU_PRECISION_INT8 ? 1 : P->precision == RGNPU_PRECISION_FP16 ? 2 : 4;
+  if (!gemm_mid_supported(pl.rows, op.out_f, op.Kpad * es, op.Kpad * es)) return false;
+  const char* e = getenv("RGNPU_MID");
+  const int mode = e ? atoi(e) : 1;
+  if (mode != 1) return mode == 2;
+  const int64_t tiles = ((pl.rows + 127) / 128) * ((op.out_f + 127) / 128);
+  const GemmChoice g = choose_gemm(pl.Mpad, op.Npad, op.Kpad * es);
+  if (P->precision == RGNPU_PRECISION_INT8)
+    return op.out_f > kNarrowMaxN && (tiles < 48 || (tiles < 128 && g.splits > 1));
+  if (op.out_f <= kNarrowMaxN || g.splits > 1) return true;
+  if (P->precision == RGNPU_PRECISION_FP16) return tiles <= 128;
+  const int64_t bm = g.kind == 2 ? 128 : 256, bn = g.kind == 0 ? 256 : 128;
+  return mid_f32_better(pl.rows, op.out_f, ((pl.rows + bm - 1) / bm) * ((op.out_f + bn - 1) / bn), bm * bn);
+}
+
 // With `scratch` the plan's buffers are views into that device array (of
 // kScratchBytes) instead of allocations of their own.
 
@@ -806,14 +840,22 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
     plan->ops[i].pool_act = act;
     for (int k = 1; k <= span; k++) plan->ops[i + k].pool_fused = true;
   }
+  // FP32 Linear -> Act: the Linear applies the activation, as the fused ops of
+  // the other precisions do (the same f32 value goes through the same
+  // function); not in capture plans, which keep the Linear's own output.
+  for (size_t i = 0; i + 1 < nops && P->precision == RGNPU_PRECISION_FP32 && !plan->capture; i++) {
+    if (P->ops[i]->kind != OP_LINEAR || P->ops[i + 1]->kind != OP_ACT || plan->ops[i].rows <= 0) continue;
+    plan->ops[i].fused_act = (int)i + 1;
+    plan->ops[i + 1].act_fused = true;
+  }
   int last = -1;
   for (size_t i = 0; i < nops; i++)
-    if (P->ops[i]->kind != OP_FLATTEN && !plan->ops[i].pool_fused) last = (int)i;
+    if (P->ops[i]->kind != OP_FLATTEN && !plan->ops[i].pool_fused && !plan->ops[i].act_fused) last = (int)i;
   int curbuf = BUF_INPUT;
   for (size_t i = 0; i < nops; i++) {
     OpPlan& pl = plan->ops[i];
     pl.in_buf = curbuf;
-    if (P->ops[i]->kind == OP_FLATTEN || pl.pool_fused) {
+    if (P->ops[i]->kind == OP_FLATTEN || pl.pool_fused || pl.act_fused) {
       pl.out_buf = curbuf;
     } else if ((int)i == last) {
       pl.out_buf = BUF_OUTPUT;
@@ -832,13 +874,14 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
     const Op& op = *P->ops[i];
     OpPlan& pl = plan->ops[i];
     if (op.kind != OP_LINEAR && op.kind != OP_CONV) continue;
+    pl.mid = use_mid(P, op, pl);
     if (P->precision != RGNPU_PRECISION_INT8) {
       // No activation quantization: binary16 (FP16) or f32 (FP32) operands,
       // the split-K workspace, and the conv's [n*L, O] GEMM output.
       if (op.diag) continue;
       const int64_t es = P->precision == RGNPU_PRECISION_FP16 ? 2 : 4;
       plan->q_bytes = std::max(plan->q_bytes, (size_t)(pl.Mpad * op.Kpad * es));
-      if (!pl.gemv && !(op.kind == OP_LINEAR && op.out_f <= kNarrowMaxN))
+      if (!pl.gemv && !pl.mid)
         plan->ws_bytes = std::max(plan->ws_bytes, gemm_workspace_bytes(pl.Mpad, op.Npad, es * op.Kpad));
       if (op.kind == OP_CONV) plan->ylo_elems = std::max(plan->ylo_elems, (size_t)(pl.rows * op.out_f));
       continue;
@@ -869,8 +912,6 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
         pl.explicit_absmax = false;
       }
     }
-    if (op.kind == OP_LINEAR && !pl.gemv && op.out_f > kNarrowMaxN)
-      plan->ws_bytes = std::max(plan->ws_bytes, gemm_workspace_bytes(pl.Mpad, op.Npad, op.Kpad));
     size_t qb = op.kind == OP_LINEAR ? (size_t)(pl.Mpad * op.Kpad) : (size_t)pl.in_len;
     plan->q_bytes = std::max(plan->q_bytes, qb);
   }
@@ -934,7 +975,7 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
   for (size_t i = 0; i < nops && P->precision == RGNPU_PRECISION_INT8 && persistent_ok; i++) {
     const Op& op = *P->ops[i];
     OpPlan& pl = plan->ops[i];
-    if (op.kind != OP_LINEAR || pl.gemv || op.out_f <= kNarrowMaxN || pl.rows <= 0 || op.out_f % 4) continue;
+    if (op.kind != OP_LINEAR || pl.gemv || pl.mid || op.out_f <= kNarrowMaxN || pl.rows <= 0 || op.out_f % 4) continue;
     if (!gemm_requant_supported(pl.Mpad, op.Npad, op.Kpad)) continue;
     size_t j = i + 1;
     while (j < nops && P->ops[j]->kind == OP_FLATTEN) j++;
@@ -961,8 +1002,9 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
   for (size_t i = 0; i < nops && P->precision == RGNPU_PRECISION_FP16 && handoff_on; i++) {
     const Op& op = *P->ops[i];
     OpPlan& pl = plan->ops[i];
-    if (op.kind != OP_LINEAR || op.diag || pl.gemv || op.out_f <= kNarrowMaxN || pl.rows <= 0 || op.out_f % 4) continue;
-    if (choose_gemm(pl.Mpad, op.Npad, 2 * op.Kpad).splits != 1) continue;
+    if (op.kind != OP_LINEAR || op.diag || pl.gemv || pl.rows <= 0) continue;
+    if (!pl.mid && (op.out_f <= kNarrowMaxN || op.out_f % 4 || choose_gemm(pl.Mpad, op.Npad, 2 * op.Kpad).splits != 1))
+      continue;
     size_t j = i + 1;
     while (j < nops && P->ops[j]->kind == OP_FLATTEN) j++;
     if (j >= nops || P->ops[j]->kind != OP_LINEAR) continue;
@@ -977,6 +1019,11 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
     cpl.q_in = pl.q_in ^ 1;
     any_requant = true;  // the second operand buffer
   }
+  // The small-tile GEMM reads exactly its rows, so the pass that makes its
+  // operand writes no padding rows (the buffer keeps room for them: a fused
+  // producer of another op on it writes its own).
+  for (size_t i = 0; i < nops; i++)
+    if (plan->ops[i].mid && !plan->ops[i].q_ready) plan->ops[i].Mpad = plan->ops[i].rows;
   // A Linear that quantizes its own input does so in one pass when the
   // shapes fit the kernel's 32-bit offsets (RGNPU_INPUT_QUANT=0, for
   // measurement: the absmax and quantize kernels instead).
@@ -1008,6 +1055,15 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
                     !pl.explicit_absmax && !pl.q_ready && !pl.requant &&
                     (pl.Mpad / 128) * (op.Npad / 128) < 128 &&
                     gemm_xq_small_supported(pl.rows, op.out_f, op.Npad, op.in_f, op.Kpad);
+      if (pl.small_xq && pl.mid) {
+        // the quantize pass (a launch and its bytes) and the small-tile GEMM
+        // instead, when that is less: every block of 16 rows and 64 columns
+        // quantizes its inputs anew, so wide outputs pay for it many times
+        double mid_us = 0.0;
+        mid_choice(0, pl.rows, op.out_f, op.Kpad, &mid_us);
+        const double pass_us = 3.5 + 1e-6 * (double)(pl.rows * op.in_f);
+        pl.small_xq = gemm_xq_small_us(pl.rows, op.Npad, op.Kpad) <= mid_us + pass_us;
+      }
       if (!pl.small_xq) continue;
       const int64_t words = gemm_xq_small_sync_words(pl.rows, op.Npad, op.Kpad);
       if (words > 0) {
@@ -1313,20 +1369,27 @@ static void enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipE
             // the GEMM reads [Mpad, Kpad] rows: an input of exactly that shape
             // on a 16-byte boundary is read in place
             const float* a = in;
-            if (pl.rows != pl.Mpad || op.K != op.Kpad || (reinterpret_cast<uintptr_t>(in) & 15) != 0) {
+            int64_t lda = op.K;
+            const bool aligned = (reinterpret_cast<uintptr_t>(in) & 15) == 0;
+            if (pl.mid ? op.K % 4 != 0 || !aligned : pl.rows != pl.Mpad || op.K != op.Kpad || !aligned) {
               float* pa = plan.q.as<float>();
               launch_pad_rows_f32(in, pl.rows, op.K, pl.Mpad, op.Kpad, pa, s);
               a = pa;
+              lda = op.Kpad;
             }
             Epilogue ep;
             ep.bias = op.d_bias.as<float>();
+            if (pl.fused_act >= 0) {
+              ep.act = P->ops[(size_t)pl.fused_act]->act;
+              ep.act_param = P->ops[(size_t)pl.fused_act]->act_param;
+            }
             ep.y = out;
             ep.y_stream = pl.out_buf == BUF_OUTPUT;
             pre = launch_events_used();
-            if (pl.gemv)
+            if (pl.mid)
+              launch_gemm_mid_f32(a, lda, lda, op.d_w.as<float>(), pl.rows, op.out_f, op.Kpad, ep, s);
+            else if (pl.gemv)
               launch_gemv_f32(a, op.d_w.as<float>(), pl.rows, op.out_f, op.Npad, op.Kpad, ep, s);
-            else if (op.out_f <= kNarrowMaxN)
-              launch_gemm_narrow_f32(a, op.d_w.as<float>(), pl.rows, op.out_f, op.Kpad, ep, s);
             else
               launch_gemm_f32(a, op.d_w.as<float>(), pl.rows, op.out_f, pl.Mpad, op.Npad, op.Kpad, ep,
                               plan.ws.as<int32_t>(), plan.ws_bytes, s);
@@ -1356,10 +1419,10 @@ static void enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipE
               ep.y = nullptr;  // nothing reads the f32 output
             }
             pre = launch_events_used();
-            if (pl.gemv)
+            if (pl.mid)
+              launch_gemm_mid_f16(h, op.d_w.as<uint16_t>(), pl.rows, op.out_f, op.Kpad, ep, s);
+            else if (pl.gemv)
               launch_gemv_f16(h, op.d_w.as<uint16_t>(), pl.rows, op.out_f, op.Npad, op.Kpad, ep, s);
-            else if (op.out_f <= kNarrowMaxN)
-              launch_gemm_narrow_f16(h, op.d_w.as<uint16_t>(), pl.rows, op.out_f, op.Kpad, ep, s);
             else
               launch_gemm_f16(h, op.d_w.as<uint16_t>(), pl.rows, op.out_f, pl.Mpad, op.Npad, op.Kpad, ep,
                               plan.ws.as<int32_t>(), plan.ws_bytes, s);
@@ -1431,11 +1494,12 @@ static void enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipE
           } else if (narrow_xq) {
             launch_gemm_narrow_xq(in, op.d_w.as<int8_t>(), pl.rows, op.out_f, op.in_f, op.Kpad, ep, cap ? qa : nullptr,
                                   cap ? scales + pl.scale_base : nullptr, s);
+          } else if (pl.mid) {
+            launch_gemm_mid(qa, op.d_w.as<int8_t>(), pl.rows, op.out_f, op.Kpad, ep, s);
           } else if (op.out_f <= kNarrowMaxN) {
             launch_gemm_narrow(qa, op.d_w.as<int8_t>(), pl.rows, op.out_f, op.Kpad, ep, s);
           } else {
-            launch_gemm(qa, op.d_w.as<int8_t>(), pl.rows, op.out_f, pl.Mpad, op.Npad, op.Kpad, ep,
-                        plan.ws.as<int32_t>(), plan.ws_bytes, s);
+            launch_gemm(qa, op.d_w.as<int8_t>(), pl.rows, op.out_f, pl.Mpad, op.Npad, op.Kpad, ep, s);
           }
         }
         if (cap) RG_HIP(hipMemcpyAsync(plan.cap_q[i]->p, qa, (size_t)(pl.Mpad * op.Kpad), hipMemcpyDeviceToDevice, s));
@@ -1589,7 +1653,7 @@ static void enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipE
         break;
       case OP_ACT:
         pre = launch_events_used();
-        if (pl.pool_fused) break;  // applied by the conv before its pool
+        if (pl.pool_fused || pl.act_fused) break;  // applied by the conv before its pool, or by the Linear
         launch_activation(in, out, pl.in_len, op.act, op.act_param, emit, s);
         break;
       case OP_AFFINE: {
@@ -1623,7 +1687,7 @@ static void enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipE
       // likewise has none of its own), or the program runs as one tiny
       // kernel (only the last op's output leaves its LDS), or the pool is
       // the first of a conv pair's (its output stays in LDS).
-      const bool has_out = !pl.requant && !pl.handoff && !pl.pool_r16 && !(pl.pool_fused && op.kind != OP_POOL) &&
+      const bool has_out = !pl.requant && !pl.handoff && !pl.pool_r16 && pl.fused_act < 0 && !(pl.pool_fused && op.kind != OP_POOL) &&
                            !(plan.tiny && pl.out_buf != BUF_OUTPUT) && !pl.no_out;
       plan.tap_out_ok[i] = has_out;
       if (has_out && pl.out_len > 0)

@@ -145,12 +145,12 @@ void launch_quant_images(const float* x, int64_t per_img, int64_t n_img, const u
                          int8_t* q, float* scales_out, hipStream_t s);
 
 // C[M,N] = A[Mpad,Kpad] . B[Npad,Kpad]^T with the fused epilogue.  Mpad and
-// Npad are multiples of 128, Kpad of 64.  Shapes with few tiles split K
-// through `ws` (i32 partial sums, gemm_workspace_bytes() bytes); without a
-// large enough workspace they run unsplit.
+// Npad are multiples of 128, Kpad of 64.
 void launch_gemm(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t Mpad,
-                 int64_t Npad, int64_t Kpad, const Epilogue& ep, int32_t* ws, int64_t ws_bytes,
-                 hipStream_t s);
+                 int64_t Npad, int64_t Kpad, const Epilogue& ep, hipStream_t s);
+// The FP16 and FP32 forms split K on shapes with few tiles through a
+// workspace of this many bytes (f32 partial sums); without one they run
+// unsplit.
 int64_t gemm_workspace_bytes(int64_t Mpad, int64_t Npad, int64_t Kpad);
 // Tile shape of the large GEMM for a padded problem: 0 = 256 x 256,
 // 1 = 256 x 128, 2 = 128 x 128; splits > 1 when K is split.
@@ -183,6 +183,24 @@ void launch_input_quant(const float* x, int64_t M, int64_t K, int64_t Mpad, int6
                         float* scale_out, uint32_t* sync, int spin_limit, uint32_t* stats, SlotClear clear,
                         hipStream_t s);
 
+// Linears on more than 8 rows with too few 128 x 128 tiles to fill the chip
+// (mid.hip): small output tiles, no K split over workgroups, the same
+// epilogue (with ep.h_out the FP16 operand hand-off).  A and B need no padded
+// rows; Kpad is B's row length (zeros past K).  INT8 and FP16 read the padded
+// operand [>= M, Kpad]; FP32 reads the input itself: rows lda floats apart of
+// K floats (K and lda multiples of 4, 16-byte aligned base).
+// mid_choice: the tile (an index) with the least estimated time, in us.
+bool gemm_mid_supported(int64_t M, int64_t N, int64_t lda_bytes, int64_t kb_bytes);
+int mid_choice(int mode, int64_t M, int64_t N, int64_t kb_bytes, double* us);
+bool mid_f32_better(int64_t M, int64_t N, int64_t big_tiles, int64_t big_area);
+void launch_gemm_mid(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t Kpad, const Epilogue& ep,
+                     hipStream_t s);
+void launch_gemm_mid_f16(const uint16_t* A, const uint16_t* B, int64_t M, int64_t N, int64_t Kpad_h,
+                         const Epilogue& ep, hipStream_t s);
+void launch_gemm_mid_f32(const float* A, int64_t lda, int64_t K, const float* B, int64_t M, int64_t N, int64_t Kpad_f,
+                         const Epilogue& ep, hipStream_t s);
+void load_mid_code_object(hipStream_t s);
+
 // Same contract for M <= 8 rows (weight-streaming GEMV).
 // INT8 Linear with N <= kNarrowMaxN outputs per row: one wave per row, the
 // weights from L1 (A [M,Kpad], B [>= N, Kpad]).
@@ -205,6 +223,7 @@ void launch_gemm_narrow_xq(const float* x, const int8_t* B, int64_t M, int64_t N
 // aligned) holds a 64-bit word per output in which the slices meet.  No
 // capture outputs.
 bool gemm_xq_small_supported(int64_t M, int64_t N, int64_t Npad, int64_t K, int64_t Kpad);
+double gemm_xq_small_us(int64_t M, int64_t Npad, int64_t Kpad);  // estimated time
 int64_t gemm_xq_small_sync_words(int64_t M, int64_t Npad, int64_t Kpad);
 void launch_gemm_xq_small(const float* x, const int8_t* B, int64_t M, int64_t N, int64_t Npad, int64_t K,
                           int64_t Kpad, const Epilogue& ep, uint32_t* sync, hipStream_t s);
@@ -231,10 +250,6 @@ struct TinyChain {
   int32_t n = 0, rows = 0;
 };
 void launch_mlp_tiny(const float* x, float* y, const TinyChain& ch, SlotClear clear, hipStream_t s);
-void launch_gemm_narrow_f16(const uint16_t* A, const uint16_t* B, int64_t M, int64_t N, int64_t Kpad_h,
-                            const Epilogue& ep, hipStream_t s);
-void launch_gemm_narrow_f32(const float* A, const float* B, int64_t M, int64_t N, int64_t Kpad_f, const Epilogue& ep,
-                            hipStream_t s);
 // INT8 GEMV for M <= 8 rows: the matrix-core form (row blocks of 16
 // weights streamed through LDS) where gemv_mfma_supported, else the dot4
 // form.  kGmvBlocks: most 16-row blocks one workgroup of the matrix-core
