@@ -240,7 +240,14 @@ struct rgnpu_program {
   // each op (rgnpu_program_set_capture(prog, RGNPU_CAPTURE_PRODUCTION)).
   bool taps = false;
   bool taps_valid = false;
-  std::vector<hipEvent_t> ev;  // run start/end + launch events
+  // Two sets of run events (start, end, launch events), used by runs in
+  // turn: a run's start may be the previous run's last launch event
+  // (enqueue_profiled).  last_event: the event that ends the last run on this
+  // stream, or null when other work followed it.
+  std::vector<hipEvent_t> ev;
+  int ev_set = 0;
+  hipEvent_t last_event = nullptr;
+  hipEvent_t prof_start = nullptr, prof_end = nullptr;  // of the pending profile
   bool profile_pending = false;
   bool have_profile = false;
   rgnpu_profile prof{};
@@ -1242,9 +1249,9 @@ static Plan& get_plan(rgnpu_program* P, const int64_t* shape, int ndim) {
   return *P->plan;
 }
 
-// Events of one run: [0], [1] bracket the run (markers, default flags; the
-// host waits on [1]); [2 ..] are launch events: the stop event of each kernel
-// the run launches, recorded by that kernel's own dispatch.  Launch events
+// Events of one run: [0], [1] are markers before and after it, where it needs
+// them; [2 ..] are launch events: the stop event of each kernel the run
+// launches, recorded by that kernel's own dispatch.  Launch events
 // skip the system-scope fence, which is not needed for timing.  A run
 // launches one fill at most plus at most kMaxLaunchesPerOp kernels per op
 // (an FP16 im2col conv with split K launches four: im2col, GEMM, split-K
@@ -1261,32 +1268,33 @@ static void create_run_event(hipEvent_t* e, size_t index_in_set) {
 }
 
 static void ensure_events(rgnpu_program* P) {
-  const size_t need = events_per_run(P);
+  const size_t need = 2 * events_per_run(P);
   while (P->ev.size() < need) {
     hipEvent_t e;
-    create_run_event(&e, P->ev.size());
+    create_run_event(&e, P->ev.size() % events_per_run(P));
     P->ev.push_back(e);
   }
 }
 
 // Per-op (op ns, kernel ns) of one run from its event set.
-static void op_times(const rgnpu_program* P, const Plan& plan, const hipEvent_t* set, size_t i, double* op_ms,
+static void op_times(const Plan& plan, hipEvent_t start, const hipEvent_t* set, size_t i, double* op_ms,
                      double* kernel_ms) {
-  auto at = [&](int idx) { return idx < 0 ? set[0] : set[2 + idx]; };
+  auto at = [&](int idx) { return idx < 0 ? start : set[2 + idx]; };
   const auto& r = plan.roles[i];
   float a = 0, b = 0;
   if (r[2] != r[0]) RG_HIP(hipEventElapsedTime(&a, at(r[0]), at(r[2])));
   if (r[2] != r[1]) RG_HIP(hipEventElapsedTime(&b, at(r[1]), at(r[2])));
   *op_ms = a;
   *kernel_ms = b;
-  (void)P;
 }
 
 // Enqueue one run; x and y are device pointers.  `ev` is one run's event set
-// (events_per_run): [0] and [1] are recorded when it is given; with `timed`
-// every kernel also records its launch event and plan.roles says which ones
-// bound each op.  A null `ev` records nothing (back-to-back throughput runs).
-static void enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEvent_t* ev, bool timed) {
+// (events_per_run): every kernel records its launch event, plan.roles says
+// which ones bound each op, and the markers [0] and [1] are recorded as asked.
+// A null `ev` records nothing (back-to-back throughput runs).  Returns the
+// number of kernels launched.
+enum { MARK_START = 1, MARK_END = 2 };
+static int enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEvent_t* ev, int marks) {
   hipStream_t s = P->stream;
   const bool f16 = P->precision == RGNPU_PRECISION_FP16;
   const bool f32 = P->precision == RGNPU_PRECISION_FP32;
@@ -1297,12 +1305,11 @@ static void enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipE
   struct SinkOff {
     ~SinkOff() { set_launch_events(nullptr, 0); }
   } sink_off;
-  timed = timed && ev;
-  set_launch_events(timed ? ev + 2 : nullptr, timed ? (int)launch_event_cap(P) : 0);
+  set_launch_events(ev ? ev + 2 : nullptr, ev ? (int)launch_event_cap(P) : 0);
   if (cap) ensure_capture_buffers(P, plan);
   if (tap) ensure_tap_buffers(P, plan);
   plan.roles.assign(P->ops.size(), std::array<int, 3>{-1, -1, -1});
-  if (ev) RG_HIP(hipEventRecord(ev[0], s));
+  if (ev && (marks & MARK_START)) RG_HIP(hipEventRecord(ev[0], s));
   if (plan.in_scratch && !plan.mask_host.empty())
     RG_HIP(hipMemcpyAsync(plan.masks.p, plan.mask_host.data(), plan.mask_host.size(), hipMemcpyHostToDevice, s));
   uint32_t* const slot_sets = plan.slots.as<uint32_t>();
@@ -1697,27 +1704,58 @@ static void enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipE
     const int end = launch_events_used();
     plan.roles[i] = {first - 1, pre - 1, end > pre ? end - 1 : pre - 1};
   }
-  if (timed && (size_t)launch_events_used() >= launch_event_cap(P))
+  const int launched = launch_events_used();
+  if (ev && (size_t)launched >= launch_event_cap(P))
     throw Error(RGNPU_ERR_INVALID, "internal: a run launched more kernels than its event budget");
   // A program with no computing op returns its input (Flatten only).
   bool any = false;
   for (auto& o : P->ops) any |= o->kind != OP_FLATTEN;
   if (!any && plan.out_len > 0)
     RG_HIP(hipMemcpyAsync(y, x, (size_t)plan.out_len * sizeof(float), hipMemcpyDeviceToDevice, s));
-  if (ev) RG_HIP(hipEventRecord(ev[1], s));
+  if (ev && (marks & MARK_END)) RG_HIP(hipEventRecord(ev[1], s));
   P->capture_valid = cap || tap;
   P->taps_valid = tap;
+  return launched;
 }
 
-static void enqueue_profiled(rgnpu_program* P, Plan& plan, const float* x, float* y) {
+// A run with its profile.  Each kernel's own dispatch records its completion;
+// a marker packet, by contrast, takes the device ~4.5 us between two runs
+// (quickstart 15.5 -> 9 us per pass, CNN 31 -> 23 us without the two of them).
+// So the last kernel's event ends the run, and a device-resident run enqueued
+// while the previous one is still under way starts at that one's end: nothing
+// else is on the stream (should it end before this run's first kernel arrives,
+// that gap, less than the enqueue takes, is counted).  A run on an idle stream, after other work
+// (`after_work`: a host copy), with copies of its own (capture) or without
+// kernels keeps its markers.
+static void enqueue_profiled(rgnpu_program* P, Plan& plan, const float* x, float* y, bool after_work) {
   ensure_events(P);
-  enqueue(P, plan, x, y, P->ev.data(), P->profiling > 0);
+  hipEvent_t* const set = P->ev.data() + (size_t)(P->ev_set ^= 1) * events_per_run(P);
+  bool mark = after_work || P->capture || P->taps || !P->last_event;
+  if (!mark) {
+    if (hipEventQuery(P->last_event) == hipErrorNotReady)
+      (void)hipGetLastError();  // the answer, not an error
+    else
+      mark = true;
+  }
+  const hipEvent_t start = mark ? set[0] : P->last_event;
+  P->last_event = nullptr;
+  P->profile_pending = false;
+  const bool copies = P->capture || P->taps;
+  const int launched = enqueue(P, plan, x, y, set, (mark ? MARK_START : 0) | (copies ? MARK_END : 0));
+  hipEvent_t end = set[1];
+  if (!copies && launched > 0)
+    end = set[2 + launched - 1];
+  else if (!copies)
+    RG_HIP(hipEventRecord(end, P->stream));
+  P->prof_start = start;
+  P->prof_end = end;
+  P->last_event = end;
   P->profile_pending = true;
 }
 
 static void finalize_profile(rgnpu_program* P) {
   if (!P->profile_pending) return;
-  RG_HIP(hipEventSynchronize(P->ev[1]));
+  RG_HIP(hipEventSynchronize(P->prof_end));
   Plan& plan = *P->plan;
   rgnpu_profile pr{};
   pr.precision = P->precision;
@@ -1726,7 +1764,7 @@ static void finalize_profile(rgnpu_program* P) {
   pr.fp32_weight_bytes = (uint64_t)P->fp32_bytes;
   pr.npu_weight_bytes = (uint64_t)P->npu_bytes;
   float ms = 0.0f;
-  RG_HIP(hipEventElapsedTime(&ms, P->ev[0], P->ev[1]));
+  RG_HIP(hipEventElapsedTime(&ms, P->prof_start, P->prof_end));
   pr.total_ns = (uint64_t)((double)ms * 1e6);
   P->records.assign(P->ops.size(), rgnpu_op_record{});
   uint64_t total_macs = 0;
@@ -1737,7 +1775,7 @@ static void finalize_profile(rgnpu_program* P) {
     total_macs += r.macs;
     if (P->profiling > 0) {
       double a = 0, b = 0;
-      op_times(P, plan, P->ev.data(), i, &a, &b);
+      op_times(plan, P->prof_start, P->ev.data() + (size_t)P->ev_set * events_per_run(P), i, &a, &b);
       r.ns = (uint64_t)(a * 1e6);
       r.kernel_ns = (uint64_t)(b * 1e6);
     }
@@ -1856,7 +1894,7 @@ static void run_host(rgnpu_program* P, const float* x, const int64_t* shape, int
   } drain{P->stream};
   if (plan.in_len > 0)
     RG_HIP(copy_to_device(P->staging, plan.host_in.p, x, (size_t)plan.in_len * sizeof(float), P->stream));
-  enqueue_profiled(P, plan, plan.host_in.as<float>(), plan.host_out.as<float>());
+  enqueue_profiled(P, plan, plan.host_in.as<float>(), plan.host_out.as<float>(), true);
   if (plan.out_len > 0)
     RG_HIP(copy_to_host(P->staging, y, plan.host_out.p, (size_t)plan.out_len * sizeof(float), P->stream));
   RG_HIP(hipMemcpyAsync(P->stats_host, P->stats.p, kStatWords * sizeof(uint32_t), hipMemcpyDeviceToHost, P->stream));
@@ -1959,7 +1997,7 @@ int rgnpu_program_run_device(rgnpu_program* P, const float* d_x, const int64_t* 
   if (!d_y) return RGNPU_OK;
   if (!d_x && plan.in_len > 0) throw Error(RGNPU_ERR_INVALID, "x is NULL");
   if (y_cap < plan.out_len) throw Error(RGNPU_ERR_CAPACITY, "output buffer too small");
-  enqueue_profiled(P, plan, d_x, d_y);
+  enqueue_profiled(P, plan, d_x, d_y, false);
   RG_API_END
 }
 
@@ -1986,7 +2024,8 @@ int rgnpu_program_run_device_noalloc(rgnpu_program* P, const float* d_x, const i
   if (!d_y) return RGNPU_OK;
   if (!d_x && plan->in_len > 0) throw Error(RGNPU_ERR_INVALID, "x is NULL");
   if (y_cap < plan->out_len) throw Error(RGNPU_ERR_CAPACITY, "output buffer too small");
-  enqueue(P, *plan, d_x, d_y, nullptr, false);
+  P->last_event = nullptr;
+  enqueue(P, *plan, d_x, d_y, nullptr, 0);
   RG_API_END
 }
 
@@ -2023,6 +2062,7 @@ int rgnpu_program_benchmark(rgnpu_program* P, const float* d_x, const int64_t* s
     P->evict.ensure(kEvictBytes + 256);
     launch_fill_u32(P->evict.as<uint32_t>(), (kEvictBytes + 256) / 4, 0u, P->stream);
   }
+  P->last_event = nullptr;
   RG_HIP(hipStreamSynchronize(P->stream));
   RG_HIP(hipEventRecord(t0, P->stream));
   for (int32_t it = 0; it < iters; it++) {
@@ -2031,7 +2071,7 @@ int rgnpu_program_benchmark(rgnpu_program* P, const float* d_x, const int64_t* s
     if (evict)
       launch_evict(P->evict.p, kEvictBytes,
                    reinterpret_cast<uint32_t*>(static_cast<char*>(P->evict.p) + kEvictBytes), P->stream);
-    enqueue(P, plan, d_x, d_y, set, per_kernel_events);
+    enqueue(P, plan, d_x, d_y, set, MARK_START | MARK_END);
   }
   RG_HIP(hipEventRecord(t1, P->stream));
   RG_HIP(hipEventSynchronize(t1));
@@ -2049,7 +2089,7 @@ int rgnpu_program_benchmark(rgnpu_program* P, const float* d_x, const int64_t* s
         double a = 0, b = 0;
         for (int32_t it = 0; it < iters; it++) {
           double x = 0, y = 0;
-          op_times(P, plan, evs.data() + per * (size_t)it, i, &x, &y);
+          op_times(plan, evs[per * (size_t)it], evs.data() + per * (size_t)it, i, &x, &y);
           a += x;
           b += y;
         }
