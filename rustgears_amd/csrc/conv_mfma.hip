@@ -1,0 +1,354 @@
+// conv_mfma.hip -- FP16 and FP32 convolutions (C k k > 32 taps or more than 64
+// output channels; the others run in conv_direct_kernel) as one implicit GEMM
+// kernel, with the MaxPool2d(2, 2) and the next Linear's operand where they
+// follow: D[channel, pixel] = W[channel, (tap, c)] . X[(tap, c), pixel].
+//
+// These layers have few pixels per image (the CNN's second conv: 16 x 16) and
+// little work per byte on the matrix cores, so the time goes to launches and
+// round trips: as im2col + GEMM + transpose + pool they took 43 us for 100
+// images (17.3 + 12.2 + 9.8 + 3.7), the im2col matrix alone 9 times the input.
+//  * A workgroup of 4 waves owns RB x XB output pixels of one image and 16, 32
+//    or 64 channels.  The input rows under its pixels are staged in LDS
+//    channel-last, 64 bytes of channels (32 binary16 or 16 f32) at a time, zeros
+//    around the image; a K step of 64 bytes is then one tap of one channel
+//    block, and every fragment is one 16-byte LDS read.
+//  * The weights lie in memory as [channel block][tap][output channel][64
+//    bytes], so a tap of a workgroup is one contiguous run that global_load_lds
+//    copies beside the band.
+//  * Both are stored with their 16-byte pieces at piece ^ ((row >> 1) & 3), the
+//    bank-conflict-free order of the large GEMM.
+//  * Pooled outputs go through LDS, so any width and height pools here.
+#include <hip/hip_ext.h>
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <stdexcept>
+
+#include "devmath.h"
+#include "gemm_core.h"
+#include "rgnpu_internal.h"
+
+namespace rgnpu {
+
+namespace cmf {
+constexpr int kWaves = 4, kThreads = kWaves * 64;
+constexpr int kGroupBytes = 36 * 1024;  // weights staged at a time: 9 taps of 64 channels
+constexpr int kMaxLds = 156 * 1024;
+}  // namespace cmf
+
+struct ConvMfmaShape {
+  int32_t C, H, W, O, OH, OW, k, stride, pad;
+  int32_t blocks_c;            // 64-byte channel blocks
+  int32_t Opad;                // output channels of the weight layout
+  int32_t RB, XB, tiles_y, tiles_x, tiles_o;
+  int32_t BR, BC;              // band rows and columns
+  int32_t TG;                  // taps staged at a time
+  uint32_t mBC, mBR, mXB, mPW; // ceil(2^32 / d): exact quotients of the indexes divided here
+  int32_t wbase;               // LDS byte offset of the weights
+  int32_t pool, PH, PW, pbw, pbh;  // pooled output, and the pooled pixels of a full tile
+};
+
+// v / d for v, d < 2^16 and m = magic_of(d) (0 stands for d = 1).
+__device__ __forceinline__ uint32_t div_by(uint32_t v, uint32_t m) { return m ? __umulhi(v, m) : v; }
+
+// The max pool's window step: NaN propagates and ties keep the earlier element
+// (kernels.rs:180-191).
+__device__ __forceinline__ float window_take(float best, float v) { return (v > best || v != v) ? v : best; }
+
+template <int MODE, int ACT, int OCF, int PN>
+__device__ __forceinline__ void conv_mfma_out(int8_t* smem, const v4i (&acc)[OCF][PN], const ConvMfmaShape& s,
+                                              const Epilogue& ep, int b, int oy0, int ox0, int o0, int wave,
+                                              int lane) {
+  constexpr int P = 64 * PN, PS = P + 4;  // PS: the 4 lane quads' rows in different banks
+  float* const stage = reinterpret_cast<float*>(smem);
+  const int64_t L = (int64_t)s.OH * s.OW;
+#pragma unroll
+  for (int n = 0; n < PN; n++) {
+    const int p = (wave * PN + n) * 16 + (lane & 15);
+    const int ry = (int)div_by((uint32_t)p, s.mXB), rx = p - ry * s.XB;
+    const bool live = ry < s.RB && oy0 + ry < s.OH && ox0 + rx < s.OW;
+    float* const yp = ep.y + (int64_t)b * s.O * L + (int64_t)(oy0 + ry) * s.OW + ox0 + rx;
+#pragma unroll
+    for (int o = 0; o < OCF; o++) {
+      const int ch = o * 16 + 4 * (lane >> 4);
+      const v4f bias = *reinterpret_cast<const v4f*>(ep.bias + o0 + ch);  // padded past O
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float v = epi_word<ACT, MODE>(acc[o][n][e], 1.0f, bias[e], ep.act_param);
+        if (s.pool)
+          stage[(ch + e) * PS + p] = v;
+        else if (live && o0 + ch + e < s.O)
+          yp[(int64_t)(o0 + ch + e) * L] = v;
+      }
+    }
+  }
+  if (!s.pool) return;
+  __syncthreads();
+  // the tile's pooled outputs, columns fastest
+  const int py0 = oy0 >> 1, px0 = ox0 >> 1;
+  const uint32_t per = (uint32_t)(s.pbh * s.pbw);
+  const int64_t PL = (int64_t)s.PH * s.PW;
+  for (int ch = threadIdx.x >> 6; ch < 16 * OCF; ch += cmf::kWaves) {
+    if (o0 + ch >= s.O) break;
+    for (uint32_t i = (uint32_t)lane; i < per; i += 64) {
+      const int ry = (int)div_by(i, s.mPW), rx = (int)i - ry * s.pbw;
+      const int py = py0 + ry, px = px0 + rx;
+      if (py >= s.PH || px >= s.PW) continue;
+      const float* const w = stage + ch * PS + 2 * ry * s.XB + 2 * rx;
+      float best = -__builtin_inff();
+      best = window_take(best, w[0]);
+      best = window_take(best, w[1]);
+      best = window_take(best, w[s.XB]);
+      best = window_take(best, w[s.XB + 1]);
+      const int64_t at = (int64_t)(o0 + ch) * PL + (int64_t)py * s.PW + px;
+      if (MODE == kModeF16 && ep.h_out)
+        ep.h_out[(int64_t)b * ep.ldh + at] = rgmath::fp16_bits(rgmath::round_fp16(best));
+      else
+        ep.y[(int64_t)b * s.O * PL + at] = best;
+    }
+  }
+}
+
+template <int MODE, int OCF, int PN>
+__global__ __launch_bounds__(cmf::kThreads) void conv_mfma_kernel(const float* __restrict__ x,
+                                                                  const int8_t* __restrict__ wt, ConvMfmaShape s,
+                                                                  Epilogue ep) {
+  using namespace cmf;
+  constexpr int E = MODE == kModeF16 ? 8 : 4;  // channels per 16-byte piece
+  extern __shared__ __attribute__((aligned(1024))) int8_t cm_smem[];
+  int8_t* const smem = cm_smem;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // tiles of one image are neighbours on one XCD (dealt round-robin)
+  const int total = (int)gridDim.x, q8 = total >> 3, rem = total & 7, xcd = (int)blockIdx.x & 7;
+  int t = (xcd < rem ? xcd * (q8 + 1) : rem * (q8 + 1) + (xcd - rem) * q8) + ((int)blockIdx.x >> 3);
+  const int to = t % s.tiles_o;
+  t /= s.tiles_o;
+  const int tx = t % s.tiles_x;
+  t /= s.tiles_x;
+  const int ty = t % s.tiles_y, b = t / s.tiles_y;
+  const int oy0 = ty * s.RB, ox0 = tx * s.XB, o0 = to * 16 * OCF;
+  const int iy0 = oy0 * s.stride - s.pad, ix0 = ox0 * s.stride - s.pad;
+  const uint32_t HW4 = (uint32_t)(s.H * s.W) * 4u;
+  const __amdgpu_buffer_rsrc_t rx = bounded_rsrc(x + (int64_t)b * s.C * s.H * s.W);
+  const int taps = s.k * s.k;
+  v4i acc[OCF][PN];
+#pragma unroll
+  for (int o = 0; o < OCF; o++)
+#pragma unroll
+    for (int n = 0; n < PN; n++) acc[o][n] = v4i{0, 0, 0, 0};
+  uint32_t pb[PN];  // band pixel under each of the lane's output pixels (0 past the tile)
+#pragma unroll
+  for (int n = 0; n < PN; n++) {
+    const int p = (wave * PN + n) * 16 + (lane & 15);
+    const int ry = (int)div_by((uint32_t)p, s.mXB), rx_ = p - ry * s.XB;
+    pb[n] = ry < s.RB ? (uint32_t)((ry * s.BC + rx_) * s.stride) : 0u;
+  }
+  const uint32_t rd = (uint32_t)((lane & 15) * 64 + (((lane >> 4) ^ lds_swz(lane & 15)) << 4));
+  const int lr = lane >> 2, lp = (lane & 3) ^ lds_swz(lane >> 2);
+  const uint32_t items = (uint32_t)(4 * s.BR * s.BC);
+  for (int cb = 0; cb < s.blocks_c; cb++) {
+    for (int t0 = 0; t0 < taps; t0 += s.TG) {
+      const int nt = min(s.TG, taps - t0);
+      // weights of taps t0 .. t0 + nt: OCF instructions of 1 KiB per tap
+      for (int j = wave; j < nt * OCF; j += kWaves) {
+        const int tt = j / OCF, o = j % OCF;
+        const int8_t* const src = wt + (((int64_t)cb * taps + t0 + tt) * s.Opad + o0 + o * 16) * 64;
+        dma16(src + (uint32_t)(lr * 64 + lp * 16), smem + s.wbase + j * 1024);
+      }
+      if (t0 == 0) {
+        // the band: 16-byte pieces of E channels of one pixel, columns fastest
+        for (uint32_t i0 = (uint32_t)tid; i0 < items; i0 += 2 * kThreads) {
+          float v[2][E];
+          uint32_t dst[2];
+#pragma unroll
+          for (int u = 0; u < 2; u++) {
+            const uint32_t i = i0 + u * kThreads < items ? i0 + u * kThreads : i0;
+            const uint32_t r = div_by(i, s.mBC), bx = i - r * (uint32_t)s.BC;
+            const uint32_t pc = div_by(r, s.mBR), by = r - pc * (uint32_t)s.BR;
+            const int iy = iy0 + (int)by, ix = ix0 + (int)bx, c = cb * 4 * E + (int)pc * E;
+            const bool in = (uint32_t)iy < (uint32_t)s.H && (uint32_t)ix < (uint32_t)s.W;
+            const uint32_t off = (uint32_t)c * HW4 + (uint32_t)(iy * s.W + ix) * 4u;
+#pragma unroll
+            for (int e = 0; e < E; e++)
+              v[u][e] = __builtin_bit_cast(
+                  float, __builtin_amdgcn_raw_buffer_load_b32(
+                             rx, (int)(in && c + e < s.C ? off + (uint32_t)e * HW4 : kDropOffset), 0, 0));
+            const uint32_t pix = by * (uint32_t)s.BC + bx;
+            dst[u] = pix * 64u + ((pc ^ ((pix >> 1) & 3u)) << 4);
+          }
+#pragma unroll
+          for (int u = 0; u < 2; u++) {
+            v4i w;
+            if constexpr (MODE == kModeF16) {
+#pragma unroll
+              for (int g = 0; g < 4; g++)
+                w[g] = (int)((uint32_t)rgmath::fp16_bits(rgmath::round_fp16(v[u][2 * g])) |
+                             ((uint32_t)rgmath::fp16_bits(rgmath::round_fp16(v[u][2 * g + 1])) << 16));
+            } else {
+#pragma unroll
+              for (int g = 0; g < 4; g++) w[g] = __float_as_int(v[u][g]);
+            }
+            *reinterpret_cast<v4i*>(smem + dst[u]) = w;
+          }
+        }
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's weight copies
+      __syncthreads();
+      int ki = t0 / s.k, kj = t0 - ki * s.k;
+      for (int tt = 0; tt < nt; tt++) {
+        const uint32_t shift = (uint32_t)(ki * s.BC + kj);
+        v4i a[OCF], f[PN];
+#pragma unroll
+        for (int n = 0; n < PN; n++) {
+          const uint32_t pix = pb[n] + shift;
+          f[n] = *reinterpret_cast<const v4i*>(smem + pix * 64u + ((((uint32_t)lane >> 4) ^ ((pix >> 1) & 3u)) << 4));
+        }
+#pragma unroll
+        for (int o = 0; o < OCF; o++)
+          a[o] = *reinterpret_cast<const v4i*>(smem + s.wbase + (tt * OCF + o) * 1024 + rd);
+#pragma unroll
+        for (int c = 0; c < (MODE == kModeF32 ? 4 : 1); c++)
+#pragma unroll
+          for (int o = 0; o < OCF; o++)
+#pragma unroll
+            for (int n = 0; n < PN; n++) {
+              const v4f d = __builtin_bit_cast(v4f, acc[o][n]);
+              if constexpr (MODE == kModeF16)
+                acc[o][n] = __builtin_bit_cast(
+                    v4i, __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a[o]),
+                                                                __builtin_bit_cast(v8h, f[n]), d, 0, 0, 0));
+              else
+                acc[o][n] = __builtin_bit_cast(
+                    v4i, __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(v4f, a[o])[c],
+                                                              __builtin_bit_cast(v4f, f[n])[c], d, 0, 0, 0));
+            }
+        if (++kj == s.k) {
+          kj = 0;
+          ki++;
+        }
+      }
+      __syncthreads();  // the reads are done before the next copies, or the pool's stage, overwrite them
+    }
+  }
+#define RG_CMF(ACTV) conv_mfma_out<MODE, ACTV, OCF, PN>(smem, acc, s, ep, b, oy0, ox0, o0, wave, lane)
+  switch (ep.act) {
+    case rgmath::ACT_RELU: RG_CMF(rgmath::ACT_RELU); break;
+    case rgmath::ACT_SIGMOID: RG_CMF(rgmath::ACT_SIGMOID); break;
+    case rgmath::ACT_TANH: RG_CMF(rgmath::ACT_TANH); break;
+    case rgmath::ACT_GELU: RG_CMF(rgmath::ACT_GELU); break;
+    case rgmath::ACT_LEAKY_RELU: RG_CMF(rgmath::ACT_LEAKY_RELU); break;
+    case rgmath::ACT_SILU: RG_CMF(rgmath::ACT_SILU); break;
+    default: RG_CMF(rgmath::ACT_NONE); break;
+  }
+#undef RG_CMF
+}
+
+// The tile of a convolution: whole output rows where they are at most 64
+// pixels wide, as many of them as 64, 128 or 256 pixels hold.  The largest of
+// those that still gives 1.5 workgroups per CU, else the smallest that fits
+// (the CNN's second conv on 100 images: 400 workgroups of 4 rows).
+struct ConvMfmaTile {
+  int ocf = 0, pn = 0;
+  ConvMfmaShape s{};
+  int64_t grid = 0;
+  size_t lds = 0;
+};
+
+// ceil(2^32 / d): m d exceeds 2^32 by less than d, so v m / 2^32 has the
+// quotient's integer part while v d < 2^32.  d = 1 wraps to 0.
+static uint32_t magic_of(int64_t d) { return (uint32_t)(((uint64_t(1) << 32) + (uint64_t)d - 1) / (uint64_t)d); }
+
+static bool conv_mfma_tile(const ConvShape& cs, bool f16, bool pool, ConvMfmaTile* out) {
+  const int64_t cpb = f16 ? 32 : 16;  // channels per 64 bytes
+  if (cs.n <= 0 || cs.OH <= 0 || cs.OW <= 0 || (pool && (cs.OH < 2 || cs.OW < 2)) ||
+      cs.C * cs.H * cs.W * 4 >= (int64_t(1) << 31) || cs.k > 64)
+    return false;
+  const int ocf = cs.O <= 16 ? 1 : cs.O <= 32 ? 2 : 4;
+  const int64_t XB = std::min<int64_t>(cs.OW, 64), ob = 16 * ocf;
+  const int64_t TG = std::max<int64_t>(1, std::min<int64_t>(cs.k * cs.k, cmf::kGroupBytes / (ob * 64)));
+  for (int pn : {4, 2, 1}) {
+    int64_t RB = std::min<int64_t>(cs.OH, 64 * pn / XB);
+    if (pool) RB &= ~int64_t(1);
+    if (RB <= 0) continue;
+    const int64_t BR = (RB - 1) * cs.stride + cs.k, BC = (XB - 1) * cs.stride + cs.k;
+    const int64_t band = (BR * BC * 64 + 1023) / 1024 * 1024;
+    // quotients by multiplication are exact while dividend * divisor < 2^32
+    if (4 * BR * BC >= 65536 || BC >= 65536 || BR >= 65536) continue;
+    const int64_t lds = std::max(band + TG * ob * 64, pool ? ob * (64 * pn + 4) * 4 : int64_t(0));
+    if (lds > cmf::kMaxLds) continue;
+    const int64_t ty = (cs.OH + RB - 1) / RB, tx = (cs.OW + XB - 1) / XB, to = (cs.O + ob - 1) / ob;
+    const int64_t grid = cs.n * ty * tx * to;
+    if (grid >= (int64_t(1) << 31)) continue;
+    ConvMfmaTile g;
+    g.ocf = ocf;
+    g.pn = pn;
+    g.grid = grid;
+    g.lds = (size_t)lds;
+    ConvMfmaShape& s = g.s;
+    s.C = (int32_t)cs.C; s.H = (int32_t)cs.H; s.W = (int32_t)cs.W; s.O = (int32_t)cs.O;
+    s.OH = (int32_t)cs.OH; s.OW = (int32_t)cs.OW; s.k = (int32_t)cs.k;
+    s.stride = (int32_t)cs.stride; s.pad = (int32_t)cs.pad;
+    s.blocks_c = (int32_t)((cs.C + cpb - 1) / cpb);
+    s.Opad = (int32_t)round_up(cs.O, kConvMfmaOPad);
+    s.RB = (int32_t)RB; s.XB = (int32_t)XB;
+    s.tiles_y = (int32_t)ty; s.tiles_x = (int32_t)tx; s.tiles_o = (int32_t)to;
+    s.BR = (int32_t)BR; s.BC = (int32_t)BC; s.TG = (int32_t)TG;
+    s.pool = pool;
+    s.PH = (int32_t)(cs.OH / 2); s.PW = (int32_t)(cs.OW / 2);
+    s.pbh = (int32_t)(RB / 2); s.pbw = (int32_t)(XB / 2);
+    s.mBC = magic_of(BC); s.mBR = magic_of(BR); s.mXB = magic_of(XB);
+    s.mPW = pool ? magic_of(XB / 2) : 0;
+    s.wbase = (int32_t)band;
+    *out = g;
+    if (grid >= 384) break;
+  }
+  return out->ocf != 0;
+}
+
+bool conv_mfma_supported(const ConvShape& cs, bool f16, bool pool) {
+  ConvMfmaTile g;
+  return conv_mfma_tile(cs, f16, pool, &g);
+}
+
+template <int MODE, int OCF, int PN>
+static void launch_cmf_t(const ConvMfmaTile& g, const float* x, const int8_t* w, const Epilogue& ep, hipStream_t s) {
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_mfma_kernel<MODE, OCF, PN>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, cmf::kMaxLds);
+  if (attr != hipSuccess) throw std::runtime_error("MFMA conv: the device refuses its LDS size");
+  RG_LAUNCH((conv_mfma_kernel<MODE, OCF, PN>), dim3((unsigned)g.grid), dim3(cmf::kThreads), (unsigned)g.lds, s, x, w,
+            g.s, ep);
+}
+
+template <int MODE, int OCF>
+static void launch_cmf(const ConvMfmaTile& g, const float* x, const int8_t* w, const Epilogue& ep, hipStream_t s) {
+  if (g.pn == 4) launch_cmf_t<MODE, OCF, 4>(g, x, w, ep, s);
+  else if (g.pn == 2) launch_cmf_t<MODE, OCF, 2>(g, x, w, ep, s);
+  else launch_cmf_t<MODE, OCF, 1>(g, x, w, ep, s);
+}
+
+void launch_conv_mfma(const float* x, const void* w, const ConvShape& cs, bool f16, bool pool, const Epilogue& ep,
+                      hipStream_t s) {
+  ConvMfmaTile g;
+  if (!conv_mfma_tile(cs, f16, pool, &g)) throw std::logic_error("MFMA conv: unsupported shape");
+  if (ep.h_out && (!f16 || !pool)) throw std::logic_error("MFMA conv: the operand hand-off is FP16 after a pool");
+  const int8_t* const wb = reinterpret_cast<const int8_t*>(w);
+  if (f16) {
+    if (g.ocf == 1) launch_cmf<kModeF16, 1>(g, x, wb, ep, s);
+    else if (g.ocf == 2) launch_cmf<kModeF16, 2>(g, x, wb, ep, s);
+    else launch_cmf<kModeF16, 4>(g, x, wb, ep, s);
+  } else {
+    if (g.ocf == 1) launch_cmf<kModeF32, 1>(g, x, wb, ep, s);
+    else if (g.ocf == 2) launch_cmf<kModeF32, 2>(g, x, wb, ep, s);
+    else launch_cmf<kModeF32, 4>(g, x, wb, ep, s);
+  }
+}
+
+// This translation unit's code object, loaded at program creation.
+__global__ void conv_mfma_load_probe_kernel() {}
+
+void load_conv_mfma_code_object(hipStream_t s) {
+  hipLaunchKernelGGL(conv_mfma_load_probe_kernel, dim3(1), dim3(64), 0, s);
+}
+
+}  // namespace rgnpu

@@ -60,6 +60,7 @@ void load_code_object(hipStream_t s) {
   hipLaunchKernelGGL(load_probe_kernel, dim3(1), dim3(64), 0, s);
   load_requant_code_object(s);
   load_mid_code_object(s);
+  load_conv_mfma_code_object(s);
 }
 
 // Reads n 16-byte words so that the memory-side cache (256 MB on MI355X)

@@ -116,6 +116,7 @@ struct Op {
   std::vector<float> bias;
   int64_t K = 0, Kpad = 0, Npad = 0;  // Kpad in bytes (INT8) or binary16 elements (FP16)
   DevBuf d_w, d_bias, d_scale;
+  DevBuf d_wt;  // FP16 / FP32 conv that is not direct: the weights in launch_conv_mfma's order
   std::string label;
 };
 
@@ -148,7 +149,8 @@ struct OpPlan {
   // kernel pair.
   int64_t iq_sync_base = -1;
   bool mid = false;  // Linear on the small-tile GEMM of mid.hip
-  // FP32 Linear -> Act: the Linear's epilogue applies the activation
+  bool cmf = false;  // FP16 / FP32 conv in one kernel (conv_mfma.hip)
+  // FP32 Linear or such a conv -> Act: its epilogue applies the activation
   // (fused_act on it; act_fused on the Act op, which launches nothing).
   int fused_act = -1;  // the Act op's index
   bool act_fused = false;
@@ -416,6 +418,26 @@ static void upload_weights_f16(Op& op, hipStream_t s) {
   RG_HIP(hipStreamSynchronize(s));
 }
 
+// Whether an FP16 or FP32 conv runs in the direct kernel (serial sums in the
+// reference's order).
+static bool conv_direct(const Op& op) { return op.K <= kDirectConvTaps && op.out_f <= 64; }
+
+// FP16 / FP32 conv weights [O, C k k] as [channel block][tap][Opad][64 bytes].
+template <class T, class F>
+static void upload_conv_mfma(Op& op, hipStream_t s, F&& convert) {
+  const int64_t per = 64 / (int64_t)sizeof(T), taps = op.k * op.k, Opad = round_up(op.out_f, kConvMfmaOPad);
+  const int64_t blocks = (op.in_f + per - 1) / per;
+  std::vector<T> w((size_t)(blocks * taps * Opad * per), T(0));
+  for (int64_t o = 0; o < op.out_f; o++)
+    for (int64_t c = 0; c < op.in_f; c++)
+      for (int64_t t = 0; t < taps; t++)
+        w[(size_t)((((c / per) * taps + t) * Opad + o) * per + c % per)] =
+            convert(op.wh[(size_t)((o * op.in_f + c) * taps + t)]);
+  op.d_wt.ensure(w.size() * sizeof(T));
+  RG_HIP(hipMemcpyAsync(op.d_wt.p, w.data(), w.size() * sizeof(T), hipMemcpyHostToDevice, s));
+  RG_HIP(hipStreamSynchronize(s));
+}
+
 static void upload_weights(Op& op, hipStream_t s) {
   // Linear: [N, K] host -> [Npad, Kpad] device, zero padded.  Conv: the
   // reference [O, C*k*k] order becomes tap-major [Opad, Kpad], kk' =
@@ -555,6 +577,8 @@ static void compile_standard(rgnpu_program* P, const std::vector<FLayer>& F) {
     }
     if (op->kind == OP_LINEAR || op->kind == OP_CONV) P->fp32_bytes += (int64_t)(f.w.size() + f.b.size()) * 4;
     if (op->kind == OP_LINEAR || op->kind == OP_CONV || op->kind == OP_AFFINE) upload_weights_f32(*op, P->stream);
+    if (op->kind == OP_CONV && !conv_direct(*op))
+      upload_conv_mfma<float>(*op, P->stream, [](float v) { return v; });
     op->label = buf;
     P->ops.push_back(std::move(op));
   }
@@ -664,6 +688,8 @@ static void compile(rgnpu_program* P, const rgnpu_layer* layers, int64_t n) {
         upload_weights_f16(*op, P->stream);
       else
         upload_weights(*op, P->stream);
+      if (f16 && op->kind == OP_CONV && !conv_direct(*op))
+        upload_conv_mfma<uint16_t>(*op, P->stream, [](float v) { return rgmath::fp16_bits(v); });
     }
     op->label = op_label(*op);
     P->ops.push_back(std::move(op));
@@ -700,8 +726,8 @@ static int64_t numel(const std::vector<int64_t>& s) {
 // (which keeps the conv's own output); INT8 on the band kernel
 // (conv_band_epilogue_pool2, when a tile width fits), FP16 and FP32 on the
 // direct conv (conv_direct_pool).  FP32 convs carry no activation: there
-// the pattern is conv, Act (ReLU or none), pool.  Returns OW / 16, or 0,
-// with *span the number of ops after the conv that it absorbs and *act the
+// the pattern is conv, Act (ReLU or none), pool.  Returns OW / 16 (1 on the
+// last of these kernels), or 0, with *span the number of ops after the conv that it absorbs and *act the
 // activation it applies.  RGNPU_CONV_POOL=0 turns the fusion off.
 static int conv_pool_fusion(const rgnpu_program* P, const std::vector<OpPlan>& plan_ops, size_t i, int* span,
                             int* act) {
@@ -717,14 +743,21 @@ static int conv_pool_fusion(const rgnpu_program* P, const std::vector<OpPlan>& p
     if (P->ops[i + 1]->kind != OP_ACT) return 0;
     a = P->ops[i + 1]->act;
   }
-  if (a != rgmath::ACT_NONE && a != rgmath::ACT_RELU) return 0;
   const ConvShape& c = plan_ops[i].cs;
+  if (plan_ops[i].cmf) {
+    // images of fewer than 128 pixels keep the pool's own kernel and the time
+    // its record reports
+    *span = (int)n;
+    *act = a;
+    return c.OH * c.OW >= 128 && conv_mfma_supported(c, !f32, true) ? 1 : 0;
+  }
+  if (a != rgmath::ACT_NONE && a != rgmath::ACT_RELU) return 0;
   if (c.OH % 2 != 0 || (c.OW != 16 && c.OW != 32) || c.n <= 0) return 0;
   const int r16 = (int)(c.OW / 16);
   *span = (int)n;
   *act = a;
   if (P->precision != RGNPU_PRECISION_INT8)  // the direct conv, as enqueue picks it
-    return plan_ops[i].rows > 0 && op.K <= kDirectConvTaps && op.out_f <= 64 ? r16 : 0;
+    return plan_ops[i].rows > 0 && conv_direct(op) ? r16 : 0;
   return conv_pool_supported(c, r16) ? r16 : 0;
 }
 
@@ -804,6 +837,10 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
         pl.full_cov = true;
         for (auto v : rm) pl.full_cov &= v != 0;
         for (auto v : cm) pl.full_cov &= v != 0;
+        if (P->precision != RGNPU_PRECISION_INT8 && pl.rows > 0 && !conv_direct(op)) {
+          const char* e = getenv("RGNPU_CONV_MFMA");  // 0: im2col + GEMM (tests, measurements)
+          pl.cmf = !(e && atoi(e) == 0) && conv_mfma_supported(pl.cs, P->precision == RGNPU_PRECISION_FP16, false);
+        }
         pl.mask_off = (int64_t)mask_host.size();
         mask_host.insert(mask_host.end(), rm.begin(), rm.end());
         mask_host.insert(mask_host.end(), cm.begin(), cm.end());
@@ -847,11 +884,13 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
     plan->ops[i].pool_act = act;
     for (int k = 1; k <= span; k++) plan->ops[i + k].pool_fused = true;
   }
-  // FP32 Linear -> Act: the Linear applies the activation, as the fused ops of
-  // the other precisions do (the same f32 value goes through the same
-  // function); not in capture plans, which keep the Linear's own output.
+  // FP32 Linear (or conv in one kernel) -> Act: the first applies the
+  // activation, as the fused ops of the other precisions do (the same f32
+  // value goes through the same function); not in capture plans, which keep
+  // the first one's own output.
   for (size_t i = 0; i + 1 < nops && P->precision == RGNPU_PRECISION_FP32 && !plan->capture; i++) {
-    if (P->ops[i]->kind != OP_LINEAR || P->ops[i + 1]->kind != OP_ACT || plan->ops[i].rows <= 0) continue;
+    if (P->ops[i]->kind != OP_LINEAR && !(plan->ops[i].cmf && !plan->ops[i].pool_r16)) continue;
+    if (P->ops[i + 1]->kind != OP_ACT || plan->ops[i].rows <= 0) continue;
     plan->ops[i].fused_act = (int)i + 1;
     plan->ops[i + 1].act_fused = true;
   }
@@ -885,7 +924,7 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
     if (P->precision != RGNPU_PRECISION_INT8) {
       // No activation quantization: binary16 (FP16) or f32 (FP32) operands,
       // the split-K workspace, and the conv's [n*L, O] GEMM output.
-      if (op.diag) continue;
+      if (op.diag || pl.cmf) continue;
       const int64_t es = P->precision == RGNPU_PRECISION_FP16 ? 2 : 4;
       plan->q_bytes = std::max(plan->q_bytes, (size_t)(pl.Mpad * op.Kpad * es));
       if (!pl.gemv && !pl.mid)
@@ -1025,6 +1064,23 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
     cpl.q_ready = true;
     cpl.q_in = pl.q_in ^ 1;
     any_requant = true;  // the second operand buffer
+  }
+  // FP16 conv + pool -> Flatten -> Linear: the pooled outputs are that Linear's
+  // operand rows (no padding columns), written as binary16.
+  for (size_t i = 0; i + 2 < nops && P->precision == RGNPU_PRECISION_FP16 && handoff_on && !plan->capture; i++) {
+    OpPlan& pl = plan->ops[i];
+    if (!pl.cmf || !pl.pool_r16) continue;
+    size_t j = i + 2;
+    while (j < nops && P->ops[j]->kind == OP_FLATTEN) j++;
+    if (j == i + 2 || j >= nops || P->ops[j]->kind != OP_LINEAR) continue;
+    const Op& cop = *P->ops[j];
+    OpPlan& cpl = plan->ops[j];
+    if (cop.diag || cop.Kpad != cop.in_f || cpl.rows != pl.cs.n || cop.in_f * cpl.rows != plan->ops[i + 1].out_len)
+      continue;
+    pl.handoff = true;
+    pl.consumer = (int)j;
+    plan->ops[i + 1].no_out = true;
+    cpl.q_ready = true;
   }
   // The small-tile GEMM reads exactly its rows, so the pass that makes its
   // operand writes no padding rows (the buffer keeps room for them: a fused
@@ -1520,9 +1576,31 @@ static int enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEv
       }
       case OP_CONV: {
         const ConvShape& c = pl.cs;
+        if (pl.cmf) {  // FP16, FP32
+          Epilogue ep;
+          ep.bias = op.d_bias.as<float>();
+          ep.act = f32 ? rgmath::ACT_NONE : op.act;
+          ep.act_param = op.act_param;
+          if (f32 && pl.pool_r16) {
+            ep.act = pl.pool_act;
+            ep.act_param = P->ops[i + 1]->act_param;
+          } else if (pl.fused_act >= 0) {
+            ep.act = P->ops[(size_t)pl.fused_act]->act;
+            ep.act_param = P->ops[(size_t)pl.fused_act]->act_param;
+          }
+          ep.y = out;
+          if (pl.handoff) {
+            const OpPlan& cpl = plan.ops[(size_t)pl.consumer];
+            ep.h_out = cpl.q_in ? plan.q_alt.as<uint16_t>() : plan.q.as<uint16_t>();
+            ep.ldh = P->ops[(size_t)pl.consumer]->Kpad;
+          }
+          pre = launch_events_used();
+          launch_conv_mfma(in, op.d_wt.p, c, f16, pl.pool_r16 != 0, ep, s);
+          break;
+        }
         if (f32) {  // mod.rs:274-290: conv2d_forward (im2col + matmul), then the bias
           pre = launch_events_used();
-          if (pl.rows > 0 && op.K <= kDirectConvTaps && op.out_f <= 64) {
+          if (pl.rows > 0 && conv_direct(op)) {
             launch_conv_direct_f32(in, op.d_w.as<float>(), op.d_bias.as<float>(), out, c, pl.pool_act,
                                    pl.pool_r16 ? (int)c.OW : 0, s);
           } else if (pl.rows > 0) {
@@ -1540,7 +1618,7 @@ static int enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEv
         }
         if (f16) {  // npu.rs:341-376: im2col, GEMM, transpose per image
           pre = launch_events_used();
-          if (pl.rows > 0 && op.K <= kDirectConvTaps && op.out_f <= 64) {
+          if (pl.rows > 0 && conv_direct(op)) {
             launch_conv_direct_f16(in, op.d_w.as<uint16_t>(), op.d_bias.as<float>(), out, c, op.act, op.act_param,
                                    pl.pool_r16 ? (int)c.OW : 0, s);
           } else if (pl.rows > 0) {

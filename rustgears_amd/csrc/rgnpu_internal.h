@@ -338,6 +338,18 @@ void launch_conv_direct_f16(const float* x, const uint16_t* w, const float* bias
                             int act, float act_param, int pool_ow, hipStream_t s);
 void launch_conv_direct_f32(const float* x, const float* w, const float* bias, float* y, const ConvShape& cs,
                             int pool_act, int pool_ow, hipStream_t s);
+// FP16 and FP32 convolutions that the direct kernel does not take, as one
+// implicit GEMM (conv_mfma.hip): y NCHW = act(round_fp16(sum + bias)) or
+// act(sum + bias) with f32 sums.  w is [channel blocks of 64 bytes][k * k][O
+// rounded up to kConvMfmaOPad][64 bytes], zero padded.  With `pool` y is the
+// output of the MaxPool2d(2, 2) that follows; FP16 then writes the operand of
+// the Linear after a Flatten instead where ep.h_out is set (rows ep.ldh apart,
+// one per image).
+constexpr int64_t kConvMfmaOPad = 64;
+bool conv_mfma_supported(const ConvShape& cs, bool f16, bool pool);
+void launch_conv_mfma(const float* x, const void* w, const ConvShape& cs, bool f16, bool pool, const Epilogue& ep,
+                      hipStream_t s);
+void load_conv_mfma_code_object(hipStream_t s);
 // Lone ChannelAffine: y = round_fp16(fl(round_fp16(x) * scale[c]) + shift[c]), c = index % C.
 void launch_affine_f16(const float* x, int64_t n, int64_t C, const float* scale, const float* shift, float* y,
                        hipStream_t s);
