@@ -31,7 +31,8 @@ COMMON = [
     "-I", os.path.join(HERE, "..", "include"),
 ]
 
-SOURCES = ["kernels.hip", "requant.hip", "mid.hip", "conv_mfma.hip", "scratch.hip", "program.cpp", "hostcopy.cpp", "rng.cpp", "rtim.cpp"]
+SOURCES = ["kernels.hip", "requant.hip", "mid.hip", "conv_mfma.hip", "conv_direct.hip",
+           "scratch.hip", "program.cpp", "hostcopy.cpp", "rng.cpp", "rtim.cpp"]
 
 
 def _compile(src: str) -> str:

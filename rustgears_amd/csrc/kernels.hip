@@ -61,6 +61,7 @@ void load_code_object(hipStream_t s) {
   load_requant_code_object(s);
   load_mid_code_object(s);
   load_conv_mfma_code_object(s);
+  load_conv_direct_code_object(s);
 }
 
 // Reads n 16-byte words so that the memory-side cache (256 MB on MI355X)
@@ -316,7 +317,7 @@ void launch_quant_rows(const float* x, int64_t M, int64_t K, int64_t Mpad, int64
 // zero padding.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ uint32_t half2_of(float a, float b) {
-  return (uint32_t)rgmath::fp16_bits(rgmath::round_fp16(a)) | ((uint32_t)rgmath::fp16_bits(rgmath::round_fp16(b)) << 16);
+  return rgmath::half_bits(a) | (rgmath::half_bits(b) << 16);
 }
 
 template <bool VEC>
@@ -421,190 +422,9 @@ __global__ __launch_bounds__(256) void nlo_to_nchw_kernel(const float* __restric
   }
 }
 
-// Direct convolution for the FP16 and FP32 providers when a window holds at
-// most kDirectConvTaps values (C * k * k: the CNN's first conv has 27).  The
-// im2col matrix would be written to HBM and fed to an MFMA tile whose
-// columns the few output channels barely fill; here one thread computes
-// every output channel of one output pixel, summing the taps serially in
-// the reference's im2col order (ch * k + ki) * k + kj, padding taps (zeros)
-// included, as fp16_gemm_fused (npu.rs:425-445) and the serial matmul of
-// conv2d_forward (kernels.rs:218-265) do.  FP16: each input is round_fp16'd
-// and each product of two binary16 values is exact in f32, so fma gives the
-// reference's multiply-then-add; the output is act(round_fp16(sum + bias)).
-// FP32: multiply, then add (no contraction); the output is sum + bias (the
-// activation is a layer of its own).  The weights of one output channel are
-// read at a wave-uniform address.
-// FP16 direct conv outputs: act(round_fp16(acc + bias)) per output channel.
-template <int ACT, int OMAX>
-__device__ __forceinline__ void conv_direct_store_f16(const float (&acc)[OMAX], const float* __restrict__ bias,
-                                                      float* yb, int64_t L, int O, float act_param) {
-#pragma unroll
-  for (int o = 0; o < OMAX; o++)
-    if (o < O) yb[(int64_t)o * L] = act_fixed<ACT>(rgmath::round_fp16(acc[o] + bias[o]), act_param);
-}
-
 // The max pool's window step: NaN propagates and ties keep the earlier
 // element (kernels.rs:180-191).
 __device__ __forceinline__ float pool_take(float best, float v) { return (v > best || v != v) ? v : best; }
-
-// Direct conv -> MaxPool2d(2, 2) (npu.rs:384-390): the outputs as in
-// conv_direct_store_f16 (FP16) or the FP32 store followed by the
-// activation op's act_fixed (FP32: conv, Act, pool), pooled in registers.  OW is 16 or 32 and OH even
-// (host-checked), so a wave's 64 pixels are whole pairs of output rows:
-// pixel p + 1 is in lane ^ 1 and p + OW in lane ^ OW.  The even-row,
-// even-column lanes take the window in the reference's order with
-// pool_take and store the pooled value; every lane takes part in the
-// shuffles (lanes past the last pixel computed a clamped one).
-template <int ACT, int OMAX, int MODE>
-__device__ __forceinline__ void conv_direct_pool(const float (&acc)[OMAX], const float* __restrict__ bias,
-                                                     float* __restrict__ y, int64_t b, int O, int OH, int OW,
-                                                     int64_t pix, bool live, float act_param) {
-  const int oy = (int)(pix / OW), ox = (int)(pix - (int64_t)oy * OW);
-  const bool lead = live && (oy & 1) == 0 && (ox & 1) == 0;
-  const int64_t PL = (int64_t)(OH >> 1) * (OW >> 1);
-  float* const yb = y + b * (int64_t)O * PL + (oy >> 1) * (OW >> 1) + (ox >> 1);
-#pragma unroll
-  for (int o = 0; o < OMAX; o++) {
-    if (o < O) {  // O is the same for the whole wave (no break: it put acc on the stack)
-      const float s = acc[o] + bias[o];
-      const float v = act_fixed<ACT>(MODE == kModeF16 ? rgmath::round_fp16(s) : s, act_param);
-      const float h = __shfl_xor(v, 1);
-      const float d = __shfl_xor(v, OW);
-      const float dh = __shfl_xor(h, OW);
-      float best = -__builtin_inff();
-      best = pool_take(best, v);
-      best = pool_take(best, h);
-      best = pool_take(best, d);
-      best = pool_take(best, dh);
-      if (lead) yb[(int64_t)o * PL] = best;
-    }
-  }
-}
-
-template <int OMAX, int MODE>
-__global__ __launch_bounds__(256) void conv_direct_kernel(const float* __restrict__ x, const void* __restrict__ wv,
-                                                          const float* __restrict__ bias, float* __restrict__ y,
-                                                          ConvShape cs, int act, float act_param, int pool2) {
-  // weights as f32, tap-major [tap][OMAX] (channels past O are zero), so a
-  // tap's weights are OMAX / 4 broadcast 16-byte LDS reads
-  __shared__ __attribute__((aligned(16))) float ws[kDirectConvTaps * OMAX];
-  const int taps = (int)(cs.C * cs.k * cs.k), O = (int)cs.O, k = (int)cs.k;
-  for (int i = threadIdx.x; i < taps * OMAX; i += blockDim.x) {
-    const int kk = i / OMAX, o = i - kk * OMAX;
-    float w = 0.0f;
-    if (o < O) {
-      if constexpr (MODE == kModeF16)
-        w = (float)reinterpret_cast<const _Float16*>(wv)[(int64_t)o * cs.Kpad + kk];
-      else
-        w = reinterpret_cast<const float*>(wv)[(int64_t)o * cs.Kpad + kk];
-    }
-    ws[i] = w;
-  }
-  __syncthreads();
-  const int64_t b = blockIdx.y;
-  const int64_t L = cs.OH * cs.OW;
-  const int64_t pix_raw = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool live = pix_raw < L;
-  if (!live && !pool2) return;
-  const int64_t pix = live ? pix_raw : L - 1;  // pooled: every lane joins the shuffles
-  const int oy = (int)(pix / cs.OW), ox = (int)(pix - (int64_t)oy * cs.OW);
-  const int iy0 = oy * (int)cs.stride - (int)cs.pad, ix0 = ox * (int)cs.stride - (int)cs.pad;
-  const int H = (int)cs.H, W = (int)cs.W;
-  const float* xb = x + b * cs.C * cs.H * cs.W;
-  float acc[OMAX];
-#pragma unroll
-  for (int o = 0; o < OMAX; o++) acc[o] = 0.0f;
-  int kk = 0;
-  for (int ch = 0; ch < (int)cs.C; ch++)
-    for (int ki = 0; ki < k; ki++) {
-      const int iy = iy0 + ki;
-      const bool row_ok = iy >= 0 && iy < H;
-      const float* xr = xb + ((int64_t)ch * H + iy) * W;
-      for (int kj = 0; kj < k; kj++, kk++) {
-        const int ix = ix0 + kj;
-        float v = (row_ok && ix >= 0 && ix < W) ? xr[ix] : 0.0f;
-        const float4* wr = reinterpret_cast<const float4*>(ws + kk * OMAX);
-        if constexpr (MODE == kModeF16) {
-          v = rgmath::round_fp16(v);
-#pragma unroll
-          for (int q = 0; q < OMAX / 4; q++) {
-            const float4 w4 = wr[q];
-            acc[4 * q] = __builtin_fmaf(v, w4.x, acc[4 * q]);
-            acc[4 * q + 1] = __builtin_fmaf(v, w4.y, acc[4 * q + 1]);
-            acc[4 * q + 2] = __builtin_fmaf(v, w4.z, acc[4 * q + 2]);
-            acc[4 * q + 3] = __builtin_fmaf(v, w4.w, acc[4 * q + 3]);
-          }
-        } else {
-#pragma unroll
-          for (int q = 0; q < OMAX / 4; q++) {
-            const float4 w4 = wr[q];
-            const float p0 = v * w4.x, p1 = v * w4.y, p2 = v * w4.z, p3 = v * w4.w;
-            acc[4 * q] = acc[4 * q] + p0;
-            acc[4 * q + 1] = acc[4 * q + 1] + p1;
-            acc[4 * q + 2] = acc[4 * q + 2] + p2;
-            acc[4 * q + 3] = acc[4 * q + 3] + p3;
-          }
-        }
-      }
-    }
-  if (pool2) {
-    if (act == rgmath::ACT_RELU)
-      conv_direct_pool<rgmath::ACT_RELU, OMAX, MODE>(acc, bias, y, b, O, (int)cs.OH, (int)cs.OW, pix, live, act_param);
-    else
-      conv_direct_pool<rgmath::ACT_NONE, OMAX, MODE>(acc, bias, y, b, O, (int)cs.OH, (int)cs.OW, pix, live, act_param);
-    return;
-  }
-  float* yb = y + b * (int64_t)O * L + pix;
-  if constexpr (MODE == kModeF16) {
-    // one activation per unrolled store loop: with the activation switch
-    // inside the loop, the accumulators ended up on the stack
-#define RG_CDS(ACTV) conv_direct_store_f16<ACTV, OMAX>(acc, bias, yb, L, O, act_param)
-    switch (act) {
-      case rgmath::ACT_RELU: RG_CDS(rgmath::ACT_RELU); break;
-      case rgmath::ACT_SIGMOID: RG_CDS(rgmath::ACT_SIGMOID); break;
-      case rgmath::ACT_TANH: RG_CDS(rgmath::ACT_TANH); break;
-      case rgmath::ACT_GELU: RG_CDS(rgmath::ACT_GELU); break;
-      case rgmath::ACT_LEAKY_RELU: RG_CDS(rgmath::ACT_LEAKY_RELU); break;
-      case rgmath::ACT_SILU: RG_CDS(rgmath::ACT_SILU); break;
-      default: RG_CDS(rgmath::ACT_NONE); break;
-    }
-#undef RG_CDS
-  } else {
-#pragma unroll
-    for (int o = 0; o < OMAX; o++)
-      if (o < O) yb[(int64_t)o * L] = acc[o] + bias[o];
-  }
-}
-
-template <int MODE>
-static void launch_conv_direct_t(const float* x, const void* w, const float* bias, float* y, const ConvShape& cs,
-                                 int act, float act_param, int pool2, hipStream_t s) {
-  if (cs.C * cs.k * cs.k > kDirectConvTaps || cs.O > 64 || cs.O <= 0)
-    throw std::logic_error("direct conv: window or output channels too large");
-  if (pool2 && ((pool2 != 16 && pool2 != 32) || cs.OW != pool2 || cs.OH % 2 != 0 ||
-                (act != rgmath::ACT_RELU && act != rgmath::ACT_NONE)))
-    throw std::logic_error("direct conv: the fused pool needs ReLU or none, even height, width 16 or 32");
-  const int64_t L = cs.OH * cs.OW;
-  if (L <= 0 || cs.n <= 0) return;
-  if (cs.n > 65535) throw std::logic_error("direct conv: too many images for one launch");
-  const dim3 grid((unsigned)((L + 255) / 256), (unsigned)cs.n);
-  if (cs.O <= 16)
-    RG_LAUNCH((conv_direct_kernel<16, MODE>), grid, dim3(256), 0, s, x, w, bias, y, cs, act, act_param, pool2);
-  else if (cs.O <= 32)
-    RG_LAUNCH((conv_direct_kernel<32, MODE>), grid, dim3(256), 0, s, x, w, bias, y, cs, act, act_param, pool2);
-  else
-    RG_LAUNCH((conv_direct_kernel<64, MODE>), grid, dim3(256), 0, s, x, w, bias, y, cs, act, act_param, pool2);
-}
-
-void launch_conv_direct_f16(const float* x, const uint16_t* w, const float* bias, float* y, const ConvShape& cs,
-                            int act, float act_param, int pool_ow, hipStream_t s) {
-  launch_conv_direct_t<kModeF16>(x, w, bias, y, cs, act, act_param, pool_ow, s);
-}
-
-void launch_conv_direct_f32(const float* x, const float* w, const float* bias, float* y, const ConvShape& cs,
-                            int pool_act, int pool_ow, hipStream_t s) {
-  launch_conv_direct_t<kModeF32>(x, w, bias, y, cs, pool_ow ? pool_act : rgmath::ACT_NONE, 0.0f, pool_ow, s);
-}
 
 void launch_nlo_to_nchw(const float* ylo, int64_t n, int64_t O, int64_t L, float* y, hipStream_t s) {
   const int64_t total = n * O * L;
@@ -863,7 +683,7 @@ __device__ __forceinline__ float big_epilogue_slab(const int32_t* slab, int rows
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 
 // The binary16 operand of an FP16 output value (what half_rows_kernel writes).
-__device__ __forceinline__ uint32_t h16(float y) { return rgmath::fp16_bits(rgmath::round_fp16(y)); }
+__device__ __forceinline__ uint32_t h16(float y) { return rgmath::half_bits(y); }
 
 // Certified GELU for the hand-off (ACT == GELU): the operand of
 // gelu(pre) is h16 of it, and h16 never decreases (as the value it encodes)

@@ -84,7 +84,7 @@ __device__ __forceinline__ float mid_epilogue(const int32_t* red, const MidShape
       if (ep.h_out) {  // the next Linear's operand, zero past N
         uint32_t h[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) h[e] = col + e < s.N ? rgmath::fp16_bits(rgmath::round_fp16(v[e])) : 0u;
+        for (int e = 0; e < 4; e++) h[e] = col + e < s.N ? rgmath::half_bits(v[e]) : 0u;
         if (col < ep.ldh)
           *reinterpret_cast<uint2*>(ep.h_out + (int64_t)row * ep.ldh + col) =
               make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));

@@ -116,7 +116,7 @@ struct Op {
   std::vector<float> bias;
   int64_t K = 0, Kpad = 0, Npad = 0;  // Kpad in bytes (INT8) or binary16 elements (FP16)
   DevBuf d_w, d_bias, d_scale;
-  DevBuf d_wt;  // FP16 / FP32 conv that is not direct: the weights in launch_conv_mfma's order
+  DevBuf d_wt;  // FP16 / FP32 conv: the weights in the order of launch_conv_direct or launch_conv_mfma
   std::string label;
 };
 
@@ -422,6 +422,16 @@ static void upload_weights_f16(Op& op, hipStream_t s) {
 // reference's order).
 static bool conv_direct(const Op& op) { return op.K <= kDirectConvTaps && op.out_f <= 64; }
 
+// Its weights [O, C k k] as f32 [kDirectConvTaps][64].
+static void upload_conv_direct(Op& op, hipStream_t s) {
+  std::vector<float> w((size_t)(kDirectConvTaps * 64), 0.0f);
+  for (int64_t o = 0; o < op.out_f; o++)
+    for (int64_t t = 0; t < op.K; t++) w[(size_t)(t * 64 + o)] = op.wh[(size_t)(o * op.K + t)];
+  op.d_wt.ensure(w.size() * sizeof(float));
+  RG_HIP(hipMemcpyAsync(op.d_wt.p, w.data(), w.size() * sizeof(float), hipMemcpyHostToDevice, s));
+  RG_HIP(hipStreamSynchronize(s));
+}
+
 // FP16 / FP32 conv weights [O, C k k] as [channel block][tap][Opad][64 bytes].
 template <class T, class F>
 static void upload_conv_mfma(Op& op, hipStream_t s, F&& convert) {
@@ -577,7 +587,9 @@ static void compile_standard(rgnpu_program* P, const std::vector<FLayer>& F) {
     }
     if (op->kind == OP_LINEAR || op->kind == OP_CONV) P->fp32_bytes += (int64_t)(f.w.size() + f.b.size()) * 4;
     if (op->kind == OP_LINEAR || op->kind == OP_CONV || op->kind == OP_AFFINE) upload_weights_f32(*op, P->stream);
-    if (op->kind == OP_CONV && !conv_direct(*op))
+    if (op->kind == OP_CONV && conv_direct(*op))
+      upload_conv_direct(*op, P->stream);
+    else if (op->kind == OP_CONV)
       upload_conv_mfma<float>(*op, P->stream, [](float v) { return v; });
     op->label = buf;
     P->ops.push_back(std::move(op));
@@ -688,7 +700,9 @@ static void compile(rgnpu_program* P, const rgnpu_layer* layers, int64_t n) {
         upload_weights_f16(*op, P->stream);
       else
         upload_weights(*op, P->stream);
-      if (f16 && op->kind == OP_CONV && !conv_direct(*op))
+      if (f16 && op->kind == OP_CONV && conv_direct(*op))
+        upload_conv_direct(*op, P->stream);
+      else if (f16 && op->kind == OP_CONV)
         upload_conv_mfma<uint16_t>(*op, P->stream, [](float v) { return rgmath::fp16_bits(v); });
     }
     op->label = op_label(*op);
@@ -757,7 +771,7 @@ static int conv_pool_fusion(const rgnpu_program* P, const std::vector<OpPlan>& p
   *span = (int)n;
   *act = a;
   if (P->precision != RGNPU_PRECISION_INT8)  // the direct conv, as enqueue picks it
-    return plan_ops[i].rows > 0 && conv_direct(op) ? r16 : 0;
+    return plan_ops[i].rows > 0 && conv_direct(op) && conv_direct_supported(c) ? r16 : 0;
   return conv_pool_supported(c, r16) ? r16 : 0;
 }
 
@@ -1600,8 +1614,8 @@ static int enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEv
         }
         if (f32) {  // mod.rs:274-290: conv2d_forward (im2col + matmul), then the bias
           pre = launch_events_used();
-          if (pl.rows > 0 && conv_direct(op)) {
-            launch_conv_direct_f32(in, op.d_w.as<float>(), op.d_bias.as<float>(), out, c, pl.pool_act,
+          if (pl.rows > 0 && conv_direct(op) && conv_direct_supported(c)) {
+            launch_conv_direct_f32(in, op.d_wt.as<float>(), op.d_bias.as<float>(), out, c, pl.pool_act,
                                    pl.pool_r16 ? (int)c.OW : 0, s);
           } else if (pl.rows > 0) {
             float* a = plan.q.as<float>();
@@ -1618,8 +1632,8 @@ static int enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEv
         }
         if (f16) {  // npu.rs:341-376: im2col, GEMM, transpose per image
           pre = launch_events_used();
-          if (pl.rows > 0 && conv_direct(op)) {
-            launch_conv_direct_f16(in, op.d_w.as<uint16_t>(), op.d_bias.as<float>(), out, c, op.act, op.act_param,
+          if (pl.rows > 0 && conv_direct(op) && conv_direct_supported(c)) {
+            launch_conv_direct_f16(in, op.d_wt.as<float>(), op.d_bias.as<float>(), out, c, op.act, op.act_param,
                                    pl.pool_r16 ? (int)c.OW : 0, s);
           } else if (pl.rows > 0) {
             uint16_t* h = plan.q.as<uint16_t>();
