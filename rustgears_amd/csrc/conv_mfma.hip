@@ -136,6 +136,10 @@ __global__ __launch_bounds__(cmf::kThreads) void conv_mfma_kernel(const float* _
   for (int o = 0; o < OCF; o++)
 #pragma unroll
     for (int n = 0; n < PN; n++) acc[o][n] = v4i{0, 0, 0, 0};
+  // FP32: each channel block is summed by itself and added to the total (60
+  // channels: 3.1e-7 against 64 bits, 6.9e-7 as one chain, im2col + GEMM 5.8e-7)
+  constexpr bool BLOCKS = MODE == kModeF32;
+  v4f tot[BLOCKS ? OCF : 1][BLOCKS ? PN : 1] = {};
   uint32_t pb[PN];  // band pixel under each of the lane's output pixels (0 past the tile)
 #pragma unroll
   for (int n = 0; n < PN; n++) {
@@ -228,6 +232,15 @@ __global__ __launch_bounds__(cmf::kThreads) void conv_mfma_kernel(const float* _
         }
       }
       __syncthreads();  // the reads are done before the next copies, or the pool's stage, overwrite them
+    }
+    if constexpr (BLOCKS) {
+#pragma unroll
+      for (int o = 0; o < OCF; o++)
+#pragma unroll
+        for (int n = 0; n < PN; n++) {
+          tot[o][n] += __builtin_bit_cast(v4f, acc[o][n]);
+          acc[o][n] = cb + 1 < s.blocks_c ? v4i{0, 0, 0, 0} : __builtin_bit_cast(v4i, tot[o][n]);
+        }
     }
   }
 #define RG_CMF(ACTV) conv_mfma_out<MODE, ACTV, OCF, PN>(smem, acc, s, ep, b, oy0, ox0, o0, wave, lane)

@@ -1249,6 +1249,10 @@ __global__ __launch_bounds__(256) void gemv_kernel(const int8_t* __restrict__ A,
         case rgmath::ACT_SILU: v = act_fixed<rgmath::ACT_SILU>(pre, ep.act_param); break;
         default: v = pre; break;
       }
+      if (MODE == kModeF16 && ep.h_out) {  // the next Linear's operand (no padding columns)
+        ep.h_out[om * ep.ldh + col] = (uint16_t)rgmath::half_bits(v);
+        continue;
+      }
       ep.y[om * N + col] = v;
       if (ep.acc_out) ep.acc_out[om * N + col] = mine;
       const uint32_t key = rgmath::absmax_key(v);

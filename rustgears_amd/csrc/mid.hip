@@ -9,8 +9,8 @@
 // workgroup of 8 waves owns a small TM x TN output tile (16 to 128 rows and
 // columns, as many tiles as CUs where that can be) and all of K.  Measured
 // against 128 x 128 tiles with split K and its epilogue kernel (us, kernels
-// only): 100 x 4096 x 4096 i8 18.3 -> 7.8, f16 22.6 -> 12.2, f32 74 -> 45;
-// 1000 x 1024 x 1024 i8 17.6 -> 5.8, f16 21.8 -> 7.4, f32 33.8 -> 22.8;
+// only): 100 x 4096 x 4096 i8 18.3 -> 7.8, f16 22.6 -> 12.2, f32 75 -> 46;
+// 1000 x 1024 x 1024 i8 17.6 -> 5.8, f16 21.8 -> 7.4, f32 33.8 -> 23.8;
 // 12 x 4096 x 4096 i8 16.2 -> 4.2 (16.8 MB of weights: 4.0 TB/s).
 //  * K is walked in stages of KS x 64 bytes per row.  The stage's rows travel
 //    global -> LDS by buffer loads with the LDS as destination, 1 KiB per
@@ -40,6 +40,7 @@ namespace rgnpu {
 
 namespace mid {
 constexpr int kWaves = 8, kThreads = kWaves * 64;
+constexpr int kFlush = 8;  // FP32: stages between additions to the total
 }  // namespace mid
 
 struct MidShape {
@@ -168,9 +169,27 @@ __global__ __launch_bounds__(mid::kThreads) void gemm_mid_kernel(const int8_t* _
         dma16_buf(rb, dst, off);
     }
   };
-  // FP32 sums the even and odd halves of a chunk apart: 2 KS chains of K / (2
-  // KS) terms each round no more than the K slices of the tile GEMM did.
-  constexpr int NA = MODE == kModeF32 ? 2 : 1;
+  // FP32 rounds every step of a sum, so long chains lose what the GEMV's and
+  // the split tiles' short ones did not: the even and odd halves of a chunk
+  // are summed apart, and every kFlush stages (64 terms) both join a total.
+  // Against 64 bits, 4 x 4096 x 14336 x 4096: 6.2e-7 without the totals, 3.3e-7
+  // in the GEMV, 2.5e-7 with them (and 3-4% of the time).
+  constexpr int NA = MODE == kModeF32 ? 2 : 1, NT = MODE == kModeF32 ? 1 : 0;
+  v4f tot[NT + 1][FW][FN];
+  if constexpr (NT)
+#pragma unroll
+    for (int i = 0; i < FW; i++)
+#pragma unroll
+      for (int j = 0; j < FN; j++) tot[0][i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  auto flush = [&](v4i (&a)[NA][FW][FN]) {
+#pragma unroll
+    for (int i = 0; i < FW; i++)
+#pragma unroll
+      for (int j = 0; j < FN; j++) {
+        tot[0][i][j] += __builtin_bit_cast(v4f, a[0][i][j]) + __builtin_bit_cast(v4f, a[NA - 1][i][j]);
+        a[0][i][j] = a[NA - 1][i][j] = v4i{0, 0, 0, 0};
+      }
+  };
   v4i acc[NA][FW][FN];
 #pragma unroll
   for (int a = 0; a < NA; a++)
@@ -214,6 +233,7 @@ __global__ __launch_bounds__(mid::kThreads) void gemm_mid_kernel(const int8_t* _
             acc[0][i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[i], bf[j], acc[0][i][j], 0, 0, 0);
           }
         }
+    if (MODE == kModeF32 && (st & (kFlush - 1)) == kFlush - 1) flush(acc);
     slot_rd = slot_rd == STAGES - 1 ? 0 : slot_rd + 1;
     slot_is = slot_is == STAGES - 1 ? 0 : slot_is + 1;
   }
@@ -223,13 +243,12 @@ __global__ __launch_bounds__(mid::kThreads) void gemm_mid_kernel(const int8_t* _
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   int32_t* const red = reinterpret_cast<int32_t*>(smem);
+  if constexpr (MODE == kModeF32) flush(acc);
 #pragma unroll
   for (int i = 0; i < FW; i++)
 #pragma unroll
     for (int j = 0; j < FN; j++) {
-      v4i sum = acc[0][i][j];
-      if constexpr (MODE == kModeF32)
-        sum = __builtin_bit_cast(v4i, __builtin_bit_cast(v4f, sum) + __builtin_bit_cast(v4f, acc[NA - 1][i][j]));
+      const v4i sum = MODE == kModeF32 ? __builtin_bit_cast(v4i, tot[0][i][j]) : acc[0][i][j];
 #pragma unroll
       for (int e = 0; e < 4; e++)
         red[(ksub * TM + (wm * FW + i) * 16 + 4 * (lane >> 4) + e) * LD + j * 16 + (lane & 15)] = sum[e];
@@ -308,17 +327,17 @@ int mid_choice(int mode, int64_t M, int64_t N, int64_t kb, double* us) {
 }
 
 // FP32 is bound by the matrix cores, so the tiles that leave the busiest CU
-// the fewest outputs win; the tile GEMM's rate per output is 9% better (1000 x
-// 4096 x 4096: 257 against 279 us), its 128 x 128 and larger tiles divide
+// the fewest outputs win; the tile GEMM's rate per output is 13% better (1000 x
+// 4096 x 4096: 257 against 290 us), its 128 x 128 and larger tiles divide
 // worse over the CUs (3000 x 4096 x 4096, 384 tiles of 256 x 128: 942 against
-// 828 us; 300 x 4096 x 4096: 252 against 120 us).
+// 873 us; 300 x 4096 x 4096: 252 against 132 us).
 bool mid_f32_better(int64_t M, int64_t N, int64_t big_tiles, int64_t big_area) {
   double mid = 0.0;
   for (const MidTile& t : kMidTiles) {
     const double u = (double)(mid_rounds(t, M, N) * t.tm * t.tn);
     if (mid == 0.0 || u < mid) mid = u;
   }
-  return 1.09 * mid < (double)((big_tiles + 255) / 256 * big_area);
+  return 1.13 * mid < (double)((big_tiles + 255) / 256 * big_area);
 }
 
 bool gemm_mid_supported(int64_t M, int64_t N, int64_t lda, int64_t kb) {

@@ -775,8 +775,8 @@ static int conv_pool_fusion(const rgnpu_program* P, const std::vector<OpPlan>& p
   return conv_pool_supported(c, r16) ? r16 : 0;
 }
 
-// Whether a Linear runs on the small-tile GEMM (mid.hip) rather than the
-// 128 x 128 and larger tiles of launch_gemm: below 128 real tiles of
+// Whether a Linear runs on the small-tile GEMM (mid.hip) rather than the GEMV
+// or the 128 x 128 and larger tiles of launch_gemm: below 128 real tiles of
 // 128 x 128 those leave CUs idle or split K (1000 x 1024 x 1024 i8: 17.6
 // against 5.8 us; above, the larger tiles load less: 1000 x 4096 x 4096 i8
 // 24.9 against 29.5 us, f16 44.4 against 51.2 us).  Exceptions:
@@ -786,13 +786,22 @@ static int conv_pool_fusion(const rgnpu_program* P, const std::vector<OpPlan>& p
 //    against 4.8 + 3.7 us).
 //  * INT8 heads of at most 16 outputs quantize as they read (launch_gemm_narrow).
 //  * FP32 is bound by the matrix cores (mid_f32_better).
+//  * FP16 and FP32 on 2 to 8 rows with 16 MB of weights or more, where the
+//    streamed weights go through LDS here and each activation row costs the
+//    GEMV another load per weight load (5 x 14336 x 4096: FP16 37.3 -> 17.6 us,
+//    FP32 67 -> 33.5; 5 x 8192 x 28672 FP16 95 -> 79). One row streams as fast
+//    in the GEMV, and smaller matrices take 3.6 us either way.
 // RGNPU_MID=0 turns it off, 2 takes it for every Linear (tests, measurements).
 static bool use_mid(const rgnpu_program* P, const Op& op, const OpPlan& pl) {
-  if (op.kind != OP_LINEAR || op.diag || pl.gemv || pl.rows <= 0) return false;
+  if (op.kind != OP_LINEAR || op.diag || pl.rows <= 0) return false;
   const int64_t es = P->precision == RGNPU_PRECISION_INT8 ? 1 : P->precision == RGNPU_PRECISION_FP16 ? 2 : 4;
   if (!gemm_mid_supported(pl.rows, op.out_f, op.Kpad * es, op.Kpad * es)) return false;
   const char* e = getenv("RGNPU_MID");
   const int mode = e ? atoi(e) : 1;
+  if (mode == 0) return false;
+  if (pl.gemv)
+    return P->precision != RGNPU_PRECISION_INT8 && pl.rows > 1 &&
+           (mode == 2 || op.out_f * op.Kpad * es >= (int64_t(16) << 20));
   if (mode != 1) return mode == 2;
   const int64_t tiles = ((pl.rows + 127) / 128) * ((op.out_f + 127) / 128);
   const GemmChoice g = choose_gemm(pl.Mpad, op.Npad, op.Kpad * es);
@@ -1053,26 +1062,26 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
     cpl.q_in = pl.q_in ^ 1;
     any_requant = true;
   }
-  // FP16: a Linear on the unsplit MFMA GEMM whose next computing op is an
-  // FP16 Linear on the same rows hands it its binary16 operand from the GEMM
-  // epilogue, so the consumer runs no conversion pass (RGNPU_F16_HANDOFF=0
-  // turns this off).
+  // FP16: a Linear (not one that splits K) whose next computing op is an FP16
+  // Linear on the same rows hands it its binary16 operand from its epilogue, so
+  // the consumer runs no conversion pass (RGNPU_F16_HANDOFF=0 turns this off).
   const char* hoff = getenv("RGNPU_F16_HANDOFF");
   const bool handoff_on = !(hoff && atoi(hoff) == 0);
   for (size_t i = 0; i < nops && P->precision == RGNPU_PRECISION_FP16 && handoff_on; i++) {
     const Op& op = *P->ops[i];
     OpPlan& pl = plan->ops[i];
-    if (op.kind != OP_LINEAR || op.diag || pl.gemv || pl.rows <= 0) continue;
-    if (!pl.mid && (op.out_f <= kNarrowMaxN || op.out_f % 4 || choose_gemm(pl.Mpad, op.Npad, 2 * op.Kpad).splits != 1))
+    if (op.kind != OP_LINEAR || op.diag || pl.rows <= 0) continue;
+    if (!pl.mid && !pl.gemv &&
+        (op.out_f <= kNarrowMaxN || op.out_f % 4 || choose_gemm(pl.Mpad, op.Npad, 2 * op.Kpad).splits != 1))
       continue;
     size_t j = i + 1;
     while (j < nops && P->ops[j]->kind == OP_FLATTEN) j++;
     if (j >= nops || P->ops[j]->kind != OP_LINEAR) continue;
     const Op& cop = *P->ops[j];
     OpPlan& cpl = plan->ops[j];
-    if (cop.diag || cop.in_f != op.out_f || cpl.rows != pl.rows || cpl.gemv || cpl.Mpad != pl.Mpad ||
-        cop.Kpad > op.Npad)
+    if (cop.diag || cop.in_f != op.out_f || cpl.rows != pl.rows || cpl.Mpad != pl.Mpad || cop.Kpad > op.Npad)
       continue;
+    if (pl.gemv && !pl.mid && cop.Kpad != op.out_f) continue;  // the GEMV writes no padding columns
     pl.handoff = true;
     pl.consumer = (int)j;
     cpl.q_ready = true;
@@ -1563,7 +1572,7 @@ static int enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEv
                            cap ? qa : nullptr, cap ? scales + pl.scale_base : nullptr,
                            pl.explicit_absmax ? clear : SlotClear{}, s);
             if (pl.explicit_absmax) first_launched();
-          } else if (pl.gemv) {
+          } else if (pl.gemv && !pl.mid) {
             launch_gemv(qa, op.d_w.as<int8_t>(), pl.rows, op.out_f, op.Npad, op.Kpad, ep, s);
           } else if (small_xq) {
             launch_gemm_xq_small(in, op.d_w.as<int8_t>(), pl.rows, op.out_f, op.Npad, op.in_f, op.Kpad, ep,
