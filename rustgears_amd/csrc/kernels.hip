@@ -897,7 +897,10 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64, OCC) void gemm_big_kernel(
   const int kbeg = (int)blockIdx.y * ks;
   const int nk = min(ks, nk_all - kbeg);
   v4i acc[FM][4];
-  big_kloop<BM, BN, WAVES_M, WAVES_N, STAGES, FM, MODE>(smem, A, B, Kpad, m0, n0, kbeg, nk, wave, wm, wn, lane, acc);
+  if constexpr (WAVES_M == 2 && WAVES_N == 4)  // never split
+    alternating_kloop<FM, STAGES, MODE>(smem, A, B, Kpad, m0, n0, nk, wave, wm, wn, lane, acc);
+  else
+    big_kloop<BM, BN, WAVES_M, WAVES_N, STAGES, FM, MODE>(smem, A, B, Kpad, m0, n0, kbeg, nk, wave, wm, wn, lane, acc);
   if (gridDim.y > 1) {
     // Split K: raw sums for splitk_epilogue_kernel (padded extent, no masks).
     const int64_t Npad = (int64_t)tiles_n * BN;
@@ -994,32 +997,50 @@ static void launch_splitk_epilogue(const int32_t* ws, int S, int64_t M, int64_t 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int OCC, int FM, int MODE>
 static void launch_big(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t Mpad, int64_t Npad,
                        int64_t Kpad, const Epilogue& ep, int splits, int32_t* ws, hipStream_t s) {
-  const int tm = (int)(Mpad / BM), tn = (int)(Npad / BN);
+  // split sums are stored over the padded extent
+  const int tm = (int)(splits > 1 ? Mpad / BM : (M + BM - 1) / BM), tn = (int)(Npad / BN);
   const int nk = (int)(Kpad / big::BK);
   const int ks = (nk + splits - 1) / splits;
   RG_LAUNCH((gemm_big_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, OCC, FM, MODE>), dim3((unsigned)(tm * tn), (unsigned)splits),
             dim3(WAVES_M * WAVES_N * 64), 0, s, A, B, M, N, Kpad, tm, tn, ep, ks, ws);
 }
 
-// Kernel choice.  Problems with at least 256 tiles of 256 x 256 (or 256 x 128)
-// fill the CUs with the large kernels; smaller ones use 128 x 128 tiles and,
-// below 128 tiles (fewer than half the CUs busy), split K over up to 512
-// blocks of at least 4 K steps each through the workspace.
-GemmChoice choose_gemm(int64_t Mpad, int64_t Npad, int64_t Kpad) {
-  if (Mpad % 256 == 0 && Npad % 256 == 0 && (Mpad / 256) * (Npad / 256) >= 256) return {0, 1};
-  if (Mpad % 256 == 0 && Npad % 128 == 0 && (Mpad / 256) * (Npad / 128) >= 256) return {1, 1};
+// Kernel choice.  Problems with at least 256 tiles of 256 x 128 take 256
+// columns and the number of rows (256, 192 or 128) whose rounds of one workgroup
+// per CU take the least time: a K step of a tile takes bm + 104 parts (one
+// round of 256 tiles, K = 4096 INT8: 54.3, 44.2 and 34.8 us; FP16 of the same
+// bytes x 2: 105, 83.3 and 64.5 us), so 3000 x 4096 runs as 256 tiles of 192 rows in
+// one round, where 384 tiles of 256 x 128 left half the CUs idle for the second
+// half (FP16, K 4096: 151 -> 106 us a layer).  Smaller problems use 128 x 128
+// tiles and, below 128 tiles (fewer than half the CUs busy), split K over up
+// to 512 blocks of at least 4 K steps each through the workspace.
+GemmChoice choose_gemm(int64_t M, int64_t Mpad, int64_t Npad, int64_t Kpad) {
+  if (Mpad % 256 == 0 && Npad % 256 == 0 && (Mpad / 256) * (Npad / 128) >= 256) {
+    int best = 0;
+    int64_t best_cost = 0;
+    for (int bm : {256, 192, 128}) {
+      const int64_t tiles_m = (M + bm - 1) / bm;
+      if (tiles_m * bm > Mpad) continue;
+      const int64_t cost = (tiles_m * (Npad / 256) + 255) / 256 * (bm + 104);
+      if (!best || cost < best_cost) {
+        best = bm;
+        best_cost = cost;
+      }
+    }
+    return {best, 256, 1};
+  }
   const int64_t tiles = (Mpad / 128) * (Npad / 128), nk = Kpad / big::BK;
-  if (tiles >= 128) return {2, 1};
+  if (tiles >= 128) return {128, 128, 1};
   int64_t S = 512 / (tiles > 0 ? tiles : 1);
   if (S > nk / 4) S = nk / 4;
   if (S < 1) S = 1;
   const int64_t ks = (nk + S - 1) / S;
-  return {2, (int)((nk + ks - 1) / ks)};
+  return {128, 128, (int)((nk + ks - 1) / ks)};
 }
 
 int64_t gemm_workspace_bytes(int64_t Mpad, int64_t Npad, int64_t Kpad) {
-  const GemmChoice g = choose_gemm(Mpad, Npad, Kpad);
-  return g.kind == 2 && g.splits > 1 ? (int64_t)g.splits * Mpad * Npad * 4 : 0;
+  const GemmChoice g = choose_gemm(Mpad, Mpad, Npad, Kpad);
+  return g.splits > 1 ? (int64_t)g.splits * Mpad * Npad * 4 : 0;
 }
 
 template <int MODE>
@@ -1027,11 +1048,14 @@ static void launch_gemm_t(const int8_t* A, const int8_t* B, int64_t M, int64_t N
                           int64_t Kpad, const Epilogue& ep, int32_t* ws, int64_t ws_bytes, hipStream_t s) {
   if (Kpad % big::BK || Mpad % 128 || Npad % 128 || Kpad <= 0)
     throw std::logic_error("GEMM operands must be padded to 128 rows and 64-byte K steps");
-  const GemmChoice g = choose_gemm(Mpad, Npad, Kpad);
-  if (g.kind == 0) {
-    launch_big<256, 256, 2, 4, 4, 1, 8, MODE>(A, B, M, N, Mpad, Npad, Kpad, ep, 1, nullptr, s);
-  } else if (g.kind == 1) {
-    launch_big<256, 128, 2, 2, 3, 2, 8, MODE>(A, B, M, N, Mpad, Npad, Kpad, ep, 1, nullptr, s);
+  const GemmChoice g = choose_gemm(M, Mpad, Npad, Kpad);
+  if (g.bn == 256) {
+    if (g.bm == 256)
+      launch_big<256, 256, 2, 4, 4, 1, 8, MODE>(A, B, M, N, Mpad, Npad, Kpad, ep, 1, nullptr, s);
+    else if (g.bm == 192)
+      launch_big<192, 256, 2, 4, 5, 1, 6, MODE>(A, B, M, N, Mpad, Npad, Kpad, ep, 1, nullptr, s);
+    else
+      launch_big<128, 256, 2, 4, 6, 1, 4, MODE>(A, B, M, N, Mpad, Npad, Kpad, ep, 1, nullptr, s);
   } else {
     if constexpr (MODE != kModeI8) {
       if (g.splits > 1 && ws && ws_bytes >= (int64_t)g.splits * Mpad * Npad * 4) {

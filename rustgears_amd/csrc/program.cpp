@@ -804,13 +804,13 @@ static bool use_mid(const rgnpu_program* P, const Op& op, const OpPlan& pl) {
            (mode == 2 || op.out_f * op.Kpad * es >= (int64_t(16) << 20));
   if (mode != 1) return mode == 2;
   const int64_t tiles = ((pl.rows + 127) / 128) * ((op.out_f + 127) / 128);
-  const GemmChoice g = choose_gemm(pl.Mpad, op.Npad, op.Kpad * es);
+  const GemmChoice g = choose_gemm(pl.rows, pl.Mpad, op.Npad, op.Kpad * es);
   if (P->precision == RGNPU_PRECISION_INT8)
     return op.out_f > kNarrowMaxN && (tiles < 48 || (tiles < 128 && g.splits > 1));
   if (op.out_f <= kNarrowMaxN || g.splits > 1) return true;
   if (P->precision == RGNPU_PRECISION_FP16) return tiles <= 128;
-  const int64_t bm = g.kind == 2 ? 128 : 256, bn = g.kind == 0 ? 256 : 128;
-  return mid_f32_better(pl.rows, op.out_f, ((pl.rows + bm - 1) / bm) * ((op.out_f + bn - 1) / bn), bm * bn);
+  return mid_f32_better(pl.rows, op.out_f, ((pl.rows + g.bm - 1) / g.bm) * ((op.out_f + g.bn - 1) / g.bn),
+                        (int64_t)g.bm * g.bn);
 }
 
 // With `scratch` the plan's buffers are views into that device array (of
@@ -1057,7 +1057,7 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
     pl.requant = true;
     pl.consumer = (int)j;
     pl.sync_base = round_up(slots, kSpreadStride);
-    slots = pl.sync_base + requant_sync_words(pl.Mpad, op.Npad, op.Kpad);
+    slots = pl.sync_base + requant_sync_words(pl.rows, pl.Mpad, op.Npad, op.Kpad);
     cpl.q_ready = true;
     cpl.q_in = pl.q_in ^ 1;
     any_requant = true;
@@ -1072,7 +1072,7 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
     OpPlan& pl = plan->ops[i];
     if (op.kind != OP_LINEAR || op.diag || pl.rows <= 0) continue;
     if (!pl.mid && !pl.gemv &&
-        (op.out_f <= kNarrowMaxN || op.out_f % 4 || choose_gemm(pl.Mpad, op.Npad, 2 * op.Kpad).splits != 1))
+        (op.out_f <= kNarrowMaxN || op.out_f % 4 || choose_gemm(pl.rows, pl.Mpad, op.Npad, 2 * op.Kpad).splits != 1))
       continue;
     size_t j = i + 1;
     while (j < nops && P->ops[j]->kind == OP_FLATTEN) j++;

@@ -283,7 +283,7 @@ __device__ __forceinline__ void quantize_kept(const v4i (&acc)[FM][4], int8_t* q
 template <int BM, int BN, int NTHREADS>
 __device__ __forceinline__ void quantize_stored_flat(const float* y, int8_t* q, int32_t ldq, int32_t m0, int32_t n0,
                                                      int32_t M, int32_t N, float inv, int tid) {
-  constexpr int C4 = BN / 4, PER = BM * C4 / NTHREADS, BATCH = PER < 16 ? PER : 16;
+  constexpr int C4 = BN / 4, PER = BM * C4 / NTHREADS, BATCH = PER % 16 == 0 ? 16 : PER % 12 == 0 ? 12 : PER;
   static_assert(PER * NTHREADS == BM * C4 && PER % BATCH == 0 && NTHREADS % C4 == 0, "tile walk");
   const __amdgpu_buffer_rsrc_t ry = bounded_rsrc(y + (int64_t)m0 * N + n0);
   const __amdgpu_buffer_rsrc_t rq = bounded_rsrc(q + (int64_t)m0 * ldq + n0);
@@ -567,7 +567,7 @@ template <int BM, int BN, int NTHREADS>
 __device__ __forceinline__ void cert_quantize_stored_flat(const float* y, int8_t* q, int32_t ldq, int32_t m0,
                                                           int32_t n0, int32_t M, int32_t N, float inv,
                                                           const CertConst& cc, CertQueue qu, int tid) {
-  constexpr int C4 = BN / 4, PER = BM * C4 / NTHREADS, BATCH = PER < 16 ? PER : 16;
+  constexpr int C4 = BN / 4, PER = BM * C4 / NTHREADS, BATCH = PER % 16 == 0 ? 16 : PER % 12 == 0 ? 12 : PER;
   static_assert(PER * NTHREADS == BM * C4 && PER % BATCH == 0 && NTHREADS % C4 == 0, "tile walk");
   const __amdgpu_buffer_rsrc_t ry = bounded_rsrc(y + (int64_t)m0 * N + n0);
   const __amdgpu_buffer_rsrc_t rq = bounded_rsrc(q + (int64_t)m0 * ldq + n0);
@@ -660,8 +660,11 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64, OCC) void gemm_requant_kern
       asm volatile("" ::: "memory");
     }
     const float4 b4 = *reinterpret_cast<const float4*>(ep.bias + n0 + wcolw + 4 * (lane & 15));  // padded to Npad
-    big_kloop<BM, BN, WAVES_M, WAVES_N, STAGES, FM, kModeI8>(smem, A, B, (int64_t)sh.nk * BK, m0, n0, 0, sh.nk, wave,
-                                                             wm, wn, lane, acc);
+    if constexpr (WAVES_M == 2 && WAVES_N == 4)
+      alternating_kloop<FM, STAGES, kModeI8>(smem, A, B, (int64_t)sh.nk * BK, m0, n0, sh.nk, wave, wm, wn, lane, acc);
+    else
+      big_kloop<BM, BN, WAVES_M, WAVES_N, STAGES, FM, kModeI8>(smem, A, B, (int64_t)sh.nk * BK, m0, n0, 0, sh.nk, wave,
+                                                               wm, wn, lane, acc);
     if (it == 0) cs = rgmath::scale_from_absmax(rgmath::bitsf(wave_max_u32(absmax_part))) * ep.w_scale;
     const LaneSpan sp = lane_span(m0 + wrow, n0 + wcolw, M, N, lane);
     float t;
@@ -774,7 +777,7 @@ static void launch_requant_act(const int8_t* A, const int8_t* B, const RequantSh
   const int64_t T = (int64_t)sh.tiles_m * sh.tiles_n;
   int64_t G = T < cap ? T : cap;
   if (G > rqk::kMaxGrid) G = rqk::kMaxGrid;
-  if (rqk::kGoBase + G * rqk::kLine > requant_sync_words(Mpad, Npad, Kpad))
+  if (rqk::kGoBase + G * rqk::kLine > requant_sync_words(sh.M, Mpad, Npad, Kpad))
     throw std::logic_error("requant: more workgroups than sync words");
   RG_LAUNCH((gemm_requant_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, OCC, FM, ACT, CAP, CERT>), dim3((unsigned)G),
             dim3(threads), 0, s, A, B, sh, ep, rq);
@@ -1179,14 +1182,13 @@ bool gemm_requant_supported(int64_t Mpad, int64_t Npad, int64_t Kpad) {
   if (Kpad % big::BK || Mpad % 128 || Npad % 128 || Kpad <= 0) return false;
   // 32-bit offsets: whole rows and 128-row spans of the f32 output and of q
   if (Mpad * Npad * 4 >= ((int64_t)1 << 31) * 64 || Npad * 4 * 128 >= ((int64_t)1 << 31)) return false;
-  return choose_gemm(Mpad, Npad, Kpad).splits == 1;
+  return choose_gemm(Mpad, Mpad, Npad, Kpad).splits == 1;
 }
 
-int64_t requant_sync_words(int64_t Mpad, int64_t Npad, int64_t Kpad) {
+int64_t requant_sync_words(int64_t M, int64_t Mpad, int64_t Npad, int64_t Kpad) {
   // the grid never exceeds the tile count or kMaxGrid
-  const GemmChoice g = choose_gemm(Mpad, Npad, Kpad);
-  const int64_t bm = g.kind == 2 ? 128 : 256, bn = g.kind == 0 ? 256 : 128;
-  int64_t T = (Mpad / bm) * (Npad / bn);
+  const GemmChoice g = choose_gemm(M, Mpad, Npad, Kpad);
+  int64_t T = ((M + g.bm - 1) / g.bm) * (Npad / g.bn);
   if (T > rqk::kMaxGrid) T = rqk::kMaxGrid;
   return rqk::kGoBase + T * rqk::kLine;
 }
@@ -1199,21 +1201,22 @@ void launch_gemm_requant(const int8_t* A, const int8_t* B, int64_t M, int64_t N,
       (reinterpret_cast<uintptr_t>(ep.y) & 15) || (reinterpret_cast<uintptr_t>(rq.q) & 15))
     throw std::logic_error("requant: absmax slot, aligned operand and output, and sync words are required");
   if (M <= 0) return;
-  const GemmChoice g = choose_gemm(Mpad, Npad, Kpad);
-  const int64_t bm = g.kind == 2 ? 128 : 256, bn = g.kind == 0 ? 256 : 128;
-  const RequantShape sh{(int32_t)M, (int32_t)N, (int32_t)rq.ldq, (int32_t)(Kpad / big::BK), (int32_t)(Mpad / bm),
-                        (int32_t)(Npad / bn)};
+  const GemmChoice g = choose_gemm(M, Mpad, Npad, Kpad);
+  const RequantShape sh{(int32_t)M, (int32_t)N, (int32_t)rq.ldq, (int32_t)(Kpad / big::BK),
+                        (int32_t)((M + g.bm - 1) / g.bm), (int32_t)(Npad / g.bn)};
   const bool cap = ep.acc_out != nullptr;
-  if (g.kind == 0) {
-    cap ? launch_requant_shape<256, 256, 2, 4, 4, 1, 8, true>(A, B, sh, Mpad, Npad, Kpad, ep, rq, s)
-        : launch_requant_shape<256, 256, 2, 4, 4, 1, 8, false>(A, B, sh, Mpad, Npad, Kpad, ep, rq, s);
-  } else if (g.kind == 1) {
-    cap ? launch_requant_shape<256, 128, 2, 2, 3, 2, 8, true>(A, B, sh, Mpad, Npad, Kpad, ep, rq, s)
-        : launch_requant_shape<256, 128, 2, 2, 3, 2, 8, false>(A, B, sh, Mpad, Npad, Kpad, ep, rq, s);
-  } else {
-    cap ? launch_requant_shape<128, 128, 2, 2, 4, 2, 4, true>(A, B, sh, Mpad, Npad, Kpad, ep, rq, s)
-        : launch_requant_shape<128, 128, 2, 2, 4, 2, 4, false>(A, B, sh, Mpad, Npad, Kpad, ep, rq, s);
-  }
+#define RG_RQS(...)                                                                              \
+  (cap ? launch_requant_shape<__VA_ARGS__, true>(A, B, sh, Mpad, Npad, Kpad, ep, rq, s)           \
+       : launch_requant_shape<__VA_ARGS__, false>(A, B, sh, Mpad, Npad, Kpad, ep, rq, s))
+  if (g.bn == 256 && g.bm == 256)
+    RG_RQS(256, 256, 2, 4, 4, 1, 8);
+  else if (g.bn == 256 && g.bm == 192)
+    RG_RQS(192, 256, 2, 4, 5, 1, 6);
+  else if (g.bn == 256)
+    RG_RQS(128, 256, 2, 4, 6, 1, 4);
+  else
+    RG_RQS(128, 128, 2, 2, 4, 2, 4);
+#undef RG_RQS
 }
 
 }  // namespace rgnpu

@@ -152,22 +152,23 @@ void launch_gemm(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t
 // workspace of this many bytes (f32 partial sums); without one they run
 // unsplit.
 int64_t gemm_workspace_bytes(int64_t Mpad, int64_t Npad, int64_t Kpad);
-// Tile shape of the large GEMM for a padded problem: 0 = 256 x 256,
-// 1 = 256 x 128, 2 = 128 x 128; splits > 1 when K is split.
+// Tile shape of the large GEMM: 256, 192 or 128 rows x 256 columns (8 waves), or
+// 128 x 128 (4 waves); splits > 1 when K is split.  The tiles of M rows cover no
+// more than Mpad.
 struct GemmChoice {
-  int kind;
+  int bm, bn;
   int splits;
 };
-GemmChoice choose_gemm(int64_t Mpad, int64_t Npad, int64_t Kpad);
+GemmChoice choose_gemm(int64_t M, int64_t Mpad, int64_t Npad, int64_t Kpad);
 
 // The same GEMM with the next Linear's quantization fused (requant.hip):
 // a persistent grid computes every tile and its fused epilogue, raises
 // ep.absmax_out, meets at a grid barrier, then quantizes its tiles into
 // rq.q with the scale of the whole output.  Only for unsplit problems
-// (choose_gemm(...).splits == 1).  ep.y receives the f32 outputs the
+// (choose_gemm(...).splits is 1).  ep.y receives the f32 outputs the
 // quantization reads back (all of them when rq.keep_f32).
 bool gemm_requant_supported(int64_t Mpad, int64_t Npad, int64_t Kpad);
-int64_t requant_sync_words(int64_t Mpad, int64_t Npad, int64_t Kpad);
+int64_t requant_sync_words(int64_t M, int64_t Mpad, int64_t Npad, int64_t Kpad);
 void launch_gemm_requant(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t Mpad, int64_t Npad,
                          int64_t Kpad, const Epilogue& ep, const Requant& rq, hipStream_t s);
 
