@@ -180,6 +180,18 @@ __device__ __forceinline__ uint32_t q8x4(v4f v, float inv) {
 
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
+// A masked 16-byte store at byte voff + row.  The row offset is in the vector
+// offset, not in the scalar one: for a store of more than 8 bytes with a scalar
+// offset register the compiler lets the next instruction overwrite the data
+// registers, and on gfx950 the store has then taken the new value of those past
+// the first (seen as float bits among captured i32 sums, where a conversion of
+// the next row followed the store at once; which code has that pair changes
+// with every change of the schedule).  Without the register it keeps the wait
+// state that other stores get.
+__device__ __forceinline__ void store16(__amdgpu_buffer_rsrc_t r, v4u v, bool ok, uint32_t voff, uint32_t row) {
+  __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)(ok ? voff + row : kDropOffset), 0, 0);
+}
+
 // Quantizes 4 values into q's row (byte offset qoff from the wave's q base):
 // rows past M and columns past N are the operand's zero padding.
 __device__ __forceinline__ void quant_store(__amdgpu_buffer_rsrc_t rq, v4f v, float inv, uint32_t qoff, uint32_t soff,
@@ -225,11 +237,8 @@ __device__ __forceinline__ float requant_epilogue(int8_t* smem, v4i (&acc)[FM][4
       amax = __builtin_fmaxf(amax, ok ? m4 : 0.0f);
       const uint32_t soff = (uint32_t)ro * row_bytes;
       if (store || CAP)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, v), ry, (int)(ok ? voff : kDropOffset),
-                                               (int)soff, 0);
-      if constexpr (CAP)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, a), bounded_rsrc(ep.acc_out + base),
-                                               (int)(ok ? voff : kDropOffset), (int)soff, 0);
+        store16(ry, __builtin_bit_cast(v4u, v), ok, voff, soff);
+      if constexpr (CAP) store16(bounded_rsrc(ep.acc_out + base), __builtin_bit_cast(v4u, a), ok, voff, soff);
       acc[i][p] = __builtin_bit_cast(v4i, v);
     }
   }
@@ -249,8 +258,7 @@ __device__ __forceinline__ void store_kept_f32(const v4i (&acc)[FM][4], float* y
     for (int p = 0; p < 4; p++) {
       const int ro = i * 16 + p * 4;
       const bool ok = ro < sp.rows_left && sp.cols_ok;
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, acc[i][p]), ry, (int)(ok ? voff : kDropOffset),
-                                             (int)((uint32_t)ro * (uint32_t)N * 4u), 0);
+      store16(ry, __builtin_bit_cast(v4u, acc[i][p]), ok, voff, (uint32_t)ro * (uint32_t)N * 4u);
     }
 }
 
@@ -464,8 +472,7 @@ __device__ __forceinline__ float cert_epilogue(int8_t* smem, v4i (&acc)[FM][4], 
       const float m4 = __builtin_fmaxf(__builtin_fmaxf(v[0], v[1]), __builtin_fmaxf(v[2], v[3]));
       xmax = __builtin_fmaxf(xmax, ok ? m4 : 0.0f);
       if (store)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, v), ry, (int)(ok ? voff : kDropOffset),
-                                               (int)((uint32_t)ro * row_bytes), 0);
+        store16(ry, __builtin_bit_cast(v4u, v), ok, voff, (uint32_t)ro * row_bytes);
       acc[i][p] = __builtin_bit_cast(v4i, v);
     }
   }
@@ -547,9 +554,8 @@ __device__ __forceinline__ void cert_quantize_kept(const v4i (&acc)[FM][4], floa
 #pragma unroll
     for (int p = 0; p < 4; p++) {
       const int ro = i * 16 + p * 4;
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, acc[i][p]), ry,
-                                             (int)(ro < sp.rows_left && lane_ok ? voff : kDropOffset),
-                                             (int)((uint32_t)ro * (uint32_t)N * 4u), 0);
+      store16(ry, __builtin_bit_cast(v4u, acc[i][p]), ro < sp.rows_left && lane_ok, voff,
+              (uint32_t)ro * (uint32_t)N * 4u);
     }
   if (!lane_ok) return;
 #pragma unroll 1
