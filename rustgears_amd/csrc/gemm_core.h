@@ -123,12 +123,11 @@ constexpr int kLdsStride = kTK + 16;
 // ---------------------------------------------------------------------------
 // Large-problem i8 GEMM.
 //
-// Every wave owns a 128 x 64 output tile built from 8 x 4
-// v_mfma_i32_16x16x64_i8 blocks (128 accumulator registers, two waves per
-// SIMD).  A block tile is BM x BN from WAVES_M x WAVES_N waves, K step 64
-// bytes.  Two shapes are used: 256 x 128 (4 waves, two workgroups per CU)
-// and 256 x 256 (8 waves, one workgroup per CU), which moves a third fewer
-// operand bytes per MAC and leaves LDS for a deeper ring.
+// Every wave owns a (16 FM) x 64 output tile built from FM x 4
+// v_mfma_i32_16x16x64_i8 blocks (FM = 8: 128 accumulator registers, two waves
+// per SIMD).  A block tile is BM x BN from WAVES_M x WAVES_N waves, K step 64
+// bytes: 256, 192 or 128 x 256 (8 waves, one workgroup per CU) or, where those
+// would leave CUs idle, 128 x 128 (4 waves); choose_gemm has the rule.
 //
 // Operand tiles move global -> LDS with global_load_lds_dwordx4 (no VGPR
 // staging) through a STAGES-deep ring: the loads for steps k+1 .. k+STAGES-1

@@ -1011,7 +1011,7 @@ static void launch_big(const int8_t* A, const int8_t* B, int64_t M, int64_t N, i
 // round of 256 tiles, K = 4096 INT8: 54.3, 44.2 and 34.8 us; FP16 of the same
 // bytes x 2: 105, 83.3 and 64.5 us), so 3000 x 4096 runs as 256 tiles of 192 rows in
 // one round, where 384 tiles of 256 x 128 left half the CUs idle for the second
-// half (FP16, K 4096: 151 -> 106 us a layer).  Smaller problems use 128 x 128
+// half (FP16, K 4096: 151 -> 113 us a layer).  Smaller problems use 128 x 128
 // tiles and, below 128 tiles (fewer than half the CUs busy), split K over up
 // to 512 blocks of at least 4 K steps each through the workspace.
 GemmChoice choose_gemm(int64_t M, int64_t Mpad, int64_t Npad, int64_t Kpad) {

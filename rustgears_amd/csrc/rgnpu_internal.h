@@ -202,7 +202,6 @@ void launch_gemm_mid_f32(const float* A, int64_t lda, int64_t K, const float* B,
                          const Epilogue& ep, hipStream_t s);
 void load_mid_code_object(hipStream_t s);
 
-// Same contract for M <= 8 rows (weight-streaming GEMV).
 // INT8 Linear with N <= kNarrowMaxN outputs per row: one wave per row, the
 // weights from L1 (A [M,Kpad], B [>= N, Kpad]).
 constexpr int64_t kNarrowMaxN = 16;
