@@ -20,7 +20,8 @@
 //    Images too wide for that load their TAPS inputs, all before the first is
 //    used (a loop that loads and uses one tap waits for memory 27 times).  The
 //    tap count is rounded up to a compiled one; the extra taps have zero weights
-//    and finite inputs, and adding +-0 changes no sum that began at +0.
+//    and zero inputs (an input there could be infinite, and Inf * 0 is NaN), and
+//    adding +0 changes no sum that began at +0.
 //  * The weights are f32, tap-major, at wave-uniform addresses: scalar loads
 //    into SGPR operands.  (Broadcast LDS reads cost the CU 8 clocks per 4
 //    weights and wave, twice the multiply-adds they feed.)
@@ -141,6 +142,7 @@ __global__ __launch_bounds__(256) void conv_direct_kernel(const float* __restric
   const bool live = pix_raw < L;
   const int pix = live ? pix_raw : L - 1;  // every lane joins the pool's exchanges
   const float* const xb = x + (int64_t)b * s.C * s.H * s.W;
+  constexpr int MIN_TAPS = TAPS == 32 ? 28 : TAPS - 8;  // fewer take a smaller TAPS
   float v[TAPS];
   if constexpr (BAND) {
     extern __shared__ __attribute__((aligned(16))) float band[];
@@ -171,8 +173,8 @@ __global__ __launch_bounds__(256) void conv_direct_kernel(const float* __restric
     int ch = 0, ki = 0, kj = 0;
 #pragma unroll
     for (int kk = 0; kk < TAPS; kk++) {
-      // taps past the last read the last one's input; their weights are 0
-      v[kk] = band[base + (ch * s.BR + ki) * s.BW + kj];
+      const float g = band[base + (ch * s.BR + ki) * s.BW + kj];  // past the last tap: that tap's input
+      v[kk] = kk < MIN_TAPS || kk < s.taps ? g : 0.0f;
       if (kk + 1 < s.taps && ++kj == s.k) {
         kj = 0;
         if (++ki == s.k) {
