@@ -112,6 +112,16 @@ __device__ __forceinline__ float epi_word(int32_t w, float cs, float b, float p)
   }
 }
 
+// Steps of a f32 sum taken from zero before they join a total.  Each addition
+// rounds to 2^-24 of what the sum holds by then, so runs of r steps of
+// `roundings` each, `steps` / r of them, err by about the root of roundings r +
+// steps / r: least at r = sqrt(steps / roundings).
+static inline int sum_run(int64_t steps, int64_t roundings) {
+  int64_t r = 1;
+  while ((2 * r + 1) * (2 * r + 1) * roundings < 4 * steps) r++;
+  return (int)r;
+}
+
 // ---------------------------------------------------------------------------
 // MFMA operand/result layout (v_mfma_i32_16x16x64_i8): lane l supplies row
 // (l%16) of A and column (l%16) of B, K bytes [16*(l/16), 16*(l/16)+16);

@@ -31,6 +31,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <stdexcept>
+#include <type_traits>
 
 #include "devmath.h"
 #include "gemm_core.h"
@@ -40,7 +41,6 @@ namespace rgnpu {
 
 namespace mid {
 constexpr int kWaves = 8, kThreads = kWaves * 64;
-constexpr int kFlush = 8;  // FP32: stages between additions to the total
 }  // namespace mid
 
 struct MidShape {
@@ -49,6 +49,7 @@ struct MidShape {
   int32_t M, N;
   int32_t tiles_m, tiles_n;
   int32_t vec;           // y rows take 16-byte stores
+  int32_t run;           // FP16, FP32: stages summed from zero before they join the total
 };
 
 // One buffer load of 16 bytes per lane into LDS, lane i at lds + 16 i; lanes
@@ -69,15 +70,19 @@ __device__ __forceinline__ float mid_epilogue(const int32_t* red, const MidShape
   for (int r = (int)threadIdx.x / Q; r < TM; r += mid::kThreads / Q) {
     const int row = m0 + r;
     if (row >= s.M) break;
-    v4i sum = *reinterpret_cast<const v4i*>(red + r * LD + c);
+    v4i p[KS];
 #pragma unroll
-    for (int k = 1; k < KS; k++) {
-      const v4i p = *reinterpret_cast<const v4i*>(red + (k * TM + r) * LD + c);
-      if constexpr (MODE == kModeI8)
-        sum += p;
-      else
-        sum = __builtin_bit_cast(v4i, __builtin_bit_cast(v4f, sum) + __builtin_bit_cast(v4f, p));
-    }
+    for (int k = 0; k < KS; k++) p[k] = *reinterpret_cast<const v4i*>(red + (k * TM + r) * LD + c);
+#pragma unroll
+    for (int d = KS / 2; d >= 1; d /= 2)  // pairwise: log2 KS roundings of a f32 sum
+#pragma unroll
+      for (int k = 0; k < d; k++) {
+        if constexpr (MODE == kModeI8)
+          p[k] += p[k + d];
+        else
+          p[k] = __builtin_bit_cast(v4i, __builtin_bit_cast(v4f, p[k]) + __builtin_bit_cast(v4f, p[k + d]));
+      }
+    const v4i sum = p[0];
     v4f v;
 #pragma unroll
     for (int e = 0; e < 4; e++) v[e] = epi_word<ACT, MODE>(sum[e], cs, b[e], ep.act_param);
@@ -169,27 +174,19 @@ __global__ __launch_bounds__(mid::kThreads) void gemm_mid_kernel(const int8_t* _
         dma16_buf(rb, dst, off);
     }
   };
-  // FP32 rounds every step of a sum, so long chains lose what the GEMV's and
-  // the split tiles' short ones did not: the even and odd halves of a chunk
-  // are summed apart, and every kFlush stages (64 terms) both join a total.
-  // Against 64 bits, 4 x 4096 x 14336 x 4096: 6.2e-7 without the totals, 3.3e-7
-  // in the GEMV, 2.5e-7 with them (and 3-4% of the time).
-  constexpr int NA = MODE == kModeF32 ? 2 : 1, NT = MODE == kModeF32 ? 1 : 0;
-  v4f tot[NT + 1][FW][FN];
-  if constexpr (NT)
-#pragma unroll
-    for (int i = 0; i < FW; i++)
-#pragma unroll
-      for (int j = 0; j < FN; j++) tot[0][i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-  auto flush = [&](v4i (&a)[NA][FW][FN]) {
-#pragma unroll
-    for (int i = 0; i < FW; i++)
-#pragma unroll
-      for (int j = 0; j < FN; j++) {
-        tot[0][i][j] += __builtin_bit_cast(v4f, a[0][i][j]) + __builtin_bit_cast(v4f, a[NA - 1][i][j]);
-        a[0][i][j] = a[NA - 1][i][j] = v4i{0, 0, 0, 0};
-      }
-  };
+  // An f32 sum rounds at every step, so long chains lose what the GEMV's and the
+  // split tiles' short ones did not: s.run stages are summed from zero (FP32:
+  // the even and odd halves of a chunk apart), then join a total; the waves'
+  // totals meet pairwise.  Against 64 bits: FP32 1000 x 1024 x 10 in runs of 8
+  // stages 1.6e-7, now 9.9e-8 (one row per wave 1.0e-7), 3 x 4096 x 14336 1.64e-7
+  // and 1.22e-7 (GEMV 1.61e-7); FP16 outputs that are not the rounded exact sum,
+  // per mille, as one chain per wave and now: 100 x 4096 x 256 1.10 and 0.66 (split
+  // K 0.75), 5 x 14336 x 4096 2.2 and 0.8 (GEMV 1.7).  A FP16 run's first stage
+  // starts from zero instead of clearing acc (1000 x 1024 x 1024: 6.9 us as one
+  // chain, 7.2; 7.7 with clears).
+  constexpr bool TOTAL = MODE != kModeI8;
+  constexpr int NA = MODE == kModeF32 ? 2 : 1;
+  v4f tot[TOTAL ? FW : 1][TOTAL ? FN : 1] = {};
   v4i acc[NA][FW][FN];
 #pragma unroll
   for (int a = 0; a < NA; a++)
@@ -202,7 +199,8 @@ __global__ __launch_bounds__(mid::kThreads) void gemm_mid_kernel(const int8_t* _
 #pragma unroll
   for (int p = 0; p < STAGES - 1; p++) issue(p, p);  // stages past the last load nothing
   int slot_rd = 0, slot_is = STAGES - 1;
-  for (int st = 0; st < nst; st++) {
+  // Stage st's products onto acc, or from zero with `first`.
+  auto stage = [&](int st, auto first) {
     wait_vmcnt<(STAGES - 2) * NI>();  // this wave's copies of stage st have landed
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -219,23 +217,47 @@ __global__ __launch_bounds__(mid::kThreads) void gemm_mid_kernel(const int8_t* _
       for (int i = 0; i < FW; i++)
 #pragma unroll
         for (int j = 0; j < FN; j++) {
-          if constexpr (MODE == kModeF16) {
-            acc[0][i][j] = __builtin_bit_cast(
-                v4i, __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, af[i]),
-                                                            __builtin_bit_cast(v8h, bf[j]),
-                                                            __builtin_bit_cast(v4f, acc[0][i][j]), 0, 0, 0));
-          } else if constexpr (MODE == kModeF32) {
+          v4i& a = acc[c & (NA - 1)][i][j];
+          const v4i from = first.value && c < NA ? v4i{0, 0, 0, 0} : a;
+          if constexpr (MODE == kModeF32) {
             const v4f fa = __builtin_bit_cast(v4f, af[i]), fb = __builtin_bit_cast(v4f, bf[j]);
-            acc[c & 1][i][j] = __builtin_bit_cast(
-                v4i,
-                __builtin_amdgcn_mfma_f32_16x16x4f32(fa[c], fb[c], __builtin_bit_cast(v4f, acc[c & 1][i][j]), 0, 0, 0));
+            a = __builtin_bit_cast(
+                v4i, __builtin_amdgcn_mfma_f32_16x16x4f32(fa[c], fb[c], __builtin_bit_cast(v4f, from), 0, 0, 0));
           } else {
-            acc[0][i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[i], bf[j], acc[0][i][j], 0, 0, 0);
+            a = mma_block<MODE>(af[i], bf[j], from);
           }
         }
-    if (MODE == kModeF32 && (st & (kFlush - 1)) == kFlush - 1) flush(acc);
     slot_rd = slot_rd == STAGES - 1 ? 0 : slot_rd + 1;
     slot_is = slot_is == STAGES - 1 ? 0 : slot_is + 1;
+  };
+  auto add_run = [&](auto zero) {
+#pragma unroll
+    for (int i = 0; i < FW; i++)
+#pragma unroll
+      for (int j = 0; j < FN; j++) {
+        v4f sum = __builtin_bit_cast(v4f, acc[0][i][j]);
+        if constexpr (NA == 2) sum += __builtin_bit_cast(v4f, acc[1][i][j]);
+        tot[i][j] += sum;
+        if constexpr (zero.value) acc[0][i][j] = acc[NA - 1][i][j] = v4i{0, 0, 0, 0};
+      }
+  };
+  if constexpr (MODE == kModeF16) {
+    for (int st = 0; st < nst;) {
+      const int end = min(st + s.run, nst);
+      stage(st, std::true_type{});
+      for (st++; st < end; st++) stage(st, std::false_type{});
+      add_run(std::false_type{});
+    }
+  } else {  // FP32 has no registers for a second form of its stage
+    int left = s.run;
+    for (int st = 0; st < nst; st++) {
+      stage(st, std::false_type{});
+      if (MODE == kModeF32 && --left == 0) {
+        add_run(std::true_type{});
+        left = s.run;
+      }
+    }
+    if constexpr (MODE == kModeF32) add_run(std::false_type{});
   }
   // every copy has landed and every wave has read its last fragments: the
   // ring's memory takes the partial tiles
@@ -243,12 +265,12 @@ __global__ __launch_bounds__(mid::kThreads) void gemm_mid_kernel(const int8_t* _
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   int32_t* const red = reinterpret_cast<int32_t*>(smem);
-  if constexpr (MODE == kModeF32) flush(acc);
 #pragma unroll
   for (int i = 0; i < FW; i++)
 #pragma unroll
     for (int j = 0; j < FN; j++) {
-      const v4i sum = MODE == kModeF32 ? __builtin_bit_cast(v4i, tot[0][i][j]) : acc[0][i][j];
+      v4i sum = acc[0][i][j];
+      if constexpr (TOTAL) sum = __builtin_bit_cast(v4i, tot[i][j]);
 #pragma unroll
       for (int e = 0; e < 4; e++)
         red[(ksub * TM + (wm * FW + i) * 16 + 4 * (lane >> 4) + e) * LD + j * 16 + (lane & 15)] = sum[e];
@@ -352,6 +374,10 @@ static void launch_mid_t(const int8_t* A, const int8_t* B, MidShape s, const Epi
   s.tiles_m = (s.M + 16 * FM - 1) / (16 * FM);
   const int64_t cols = ep.h_out && ep.ldh > s.N ? ep.ldh : s.N;  // the operand's zero columns too
   s.tiles_n = (int32_t)((cols + 16 * FN - 1) / (16 * FN));
+  // Wide FP32 layers: 8 stages, more of them a total's addition; where the
+  // GEMV or the one-row-per-wave heads summed in shorter chains, the best.
+  const int64_t stages = (s.kb + 64 * KS - 1) / (64 * KS);
+  s.run = MODE == kModeF16 ? sum_run(stages, 3) : s.N <= kNarrowMaxN || s.M <= 8 ? sum_run(stages, 10) : 8;
   RG_LAUNCH((gemm_mid_kernel<MODE, FM, FN, KS, STAGES>), dim3((unsigned)((int64_t)s.tiles_m * s.tiles_n)),
             dim3(mid::kThreads), 0, st, A, B, s, ep);
 }
@@ -363,7 +389,8 @@ static void launch_mid_mode(const int8_t* A, int64_t lda, int64_t ka, const int8
     throw std::logic_error("mid GEMM: unsupported shape or unaligned operand");
   if (ep.h_out && (ep.ldh % 4 || MODE != kModeF16)) throw std::logic_error("mid GEMM: operand hand-off is FP16 only");
   const MidShape s{lda,        (int32_t)ka, (int32_t)kb, (int32_t)M,
-                   (int32_t)N, 0,           0,           N % 4 == 0 && (reinterpret_cast<uintptr_t>(ep.y) & 15) == 0};
+                   (int32_t)N, 0,           0,           N % 4 == 0 && (reinterpret_cast<uintptr_t>(ep.y) & 15) == 0,
+                   1};
   switch (mid_choice(MODE, M, N, kb, nullptr)) {
     case 0: launch_mid_t<MODE, 1, 1, 8, 6>(A, B, s, ep, st); break;
     case 1: launch_mid_t<MODE, 1, 2, 8, 5>(A, B, s, ep, st); break;
