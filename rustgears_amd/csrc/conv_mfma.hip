@@ -18,13 +18,14 @@
 //  * Both are stored with their 16-byte pieces at piece ^ ((row >> 1) & 3), the
 //    bank-conflict-free order of the large GEMM.
 //  * Pooled outputs go through LDS, so any width and height pools here.
-// Now 9.0 us for those 100 images (15.0 before the branch-free half_bits, with a
-// wave per channel in the pool), FP32 on 256 images 30.4 us.
+// Now 8.8 us for those 100 images (15.0 before the branch-free half_bits, with a
+// wave per channel in the pool), FP32 on 256 images 27.5 us.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <stdexcept>
+#include <type_traits>
 
 #include "devmath.h"
 #include "gemm_core.h"
@@ -58,7 +59,7 @@ __device__ __forceinline__ uint32_t div_by(uint32_t v, uint32_t m) { return m ? 
 __device__ __forceinline__ float window_take(float best, float v) { return (v > best || v != v) ? v : best; }
 
 template <int MODE, int ACT, int OCF, int PN>
-__device__ __forceinline__ void conv_mfma_out(int8_t* smem, const v4i (&acc)[OCF][PN], const ConvMfmaShape& s,
+__device__ __forceinline__ void conv_mfma_out(int8_t* smem, const v4f (&sum)[OCF][PN], const ConvMfmaShape& s,
                                               const Epilogue& ep, int b, int oy0, int ox0, int o0, int wave,
                                               int lane) {
   constexpr int P = 64 * PN, PS = P + 4;  // PS: the 4 lane quads' rows in different banks
@@ -76,7 +77,7 @@ __device__ __forceinline__ void conv_mfma_out(int8_t* smem, const v4i (&acc)[OCF
       const v4f bias = *reinterpret_cast<const v4f*>(ep.bias + o0 + ch);  // padded past O
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        const float v = epi_word<ACT, MODE>(acc[o][n][e], 1.0f, bias[e], ep.act_param);
+        const float v = epi_word<ACT, MODE>(__float_as_int(sum[o][n][e]), 1.0f, bias[e], ep.act_param);
         if (s.pool)
           stage[(ch + e) * PS + p] = v;
         else if (live && o0 + ch + e < s.O)
@@ -110,7 +111,7 @@ __device__ __forceinline__ void conv_mfma_out(int8_t* smem, const v4i (&acc)[OCF
 }
 
 template <int MODE, int OCF, int PN>
-__global__ __launch_bounds__(cmf::kThreads) void conv_mfma_kernel(const float* __restrict__ x,
+__global__ __launch_bounds__(cmf::kThreads, 2) void conv_mfma_kernel(const float* __restrict__ x,
                                                                   const int8_t* __restrict__ wt, ConvMfmaShape s,
                                                                   Epilogue ep) {
   using namespace cmf;
@@ -131,15 +132,15 @@ __global__ __launch_bounds__(cmf::kThreads) void conv_mfma_kernel(const float* _
   const uint32_t HW4 = (uint32_t)(s.H * s.W) * 4u;
   const __amdgpu_buffer_rsrc_t rx = bounded_rsrc(x + (int64_t)b * s.C * s.H * s.W);
   const int taps = s.k * s.k;
-  v4i acc[OCF][PN];
-#pragma unroll
-  for (int o = 0; o < OCF; o++)
-#pragma unroll
-    for (int n = 0; n < PN; n++) acc[o][n] = v4i{0, 0, 0, 0};
-  // FP32: each channel block is summed by itself and added to the total (60
-  // channels: 3.1e-7 against 64 bits, 6.9e-7 as one chain, im2col + GEMM 5.8e-7)
-  constexpr bool BLOCKS = MODE == kModeF32;
-  v4f tot[BLOCKS ? OCF : 1][BLOCKS ? PN : 1] = {};
+  // A chain over all of K rounds at every step, so runs of taps are summed from
+  // zero and then join a total: FP32 three taps (48 products), FP16 nine, the
+  // even and odd ones apart (its MFMA adds 32 products with fewer roundings).
+  // Against 64 bits, one chain (in FP32 per channel block) and now, in 2^-24 of
+  // the sum: FP32 32 channels 3 x 3 3.9 and 2.2 (im2col + split K 3.0), 16 channels
+  // 7 x 7 7.9 and 2.6 (2.9); FP16 60 channels 3 x 3 2.6
+  // and 1.4 (1.5).
+  constexpr int NA = MODE == kModeF16 ? 2 : 1;
+  v4f tot[OCF][PN] = {};
   uint32_t pb[PN];  // band pixel under each of the lane's output pixels (0 past the tile)
 #pragma unroll
   for (int n = 0; n < PN; n++) {
@@ -198,8 +199,9 @@ __global__ __launch_bounds__(cmf::kThreads) void conv_mfma_kernel(const float* _
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's weight copies
       __syncthreads();
       int ki = t0 / s.k, kj = t0 - ki * s.k;
-#pragma unroll 3
-      for (int tt = 0; tt < nt; tt++) {
+      v4f acc[NA][OCF][PN];
+      // Tap tt's products onto a sum, or from zero with `first`.
+      auto tap = [&](int tt, v4f (&to)[OCF][PN], auto first) {
         const uint32_t shift = (uint32_t)(ki * s.BC + kj);
         v4i a[OCF], f[PN];
 #pragma unroll
@@ -216,34 +218,63 @@ __global__ __launch_bounds__(cmf::kThreads) void conv_mfma_kernel(const float* _
           for (int o = 0; o < OCF; o++)
 #pragma unroll
             for (int n = 0; n < PN; n++) {
-              const v4f d = __builtin_bit_cast(v4f, acc[o][n]);
+              const v4f from = first.value && c == 0 ? v4f{0.0f, 0.0f, 0.0f, 0.0f} : to[o][n];
               if constexpr (MODE == kModeF16)
-                acc[o][n] = __builtin_bit_cast(
-                    v4i, __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a[o]),
-                                                                __builtin_bit_cast(v8h, f[n]), d, 0, 0, 0));
+                to[o][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a[o]),
+                                                                   __builtin_bit_cast(v8h, f[n]), from, 0, 0, 0);
               else
-                acc[o][n] = __builtin_bit_cast(
-                    v4i, __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(v4f, a[o])[c],
-                                                              __builtin_bit_cast(v4f, f[n])[c], d, 0, 0, 0));
+                to[o][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(v4f, a[o])[c],
+                                                                 __builtin_bit_cast(v4f, f[n])[c], from, 0, 0, 0);
             }
         if (++kj == s.k) {
           kj = 0;
           ki++;
         }
+      };
+      auto add_run = [&] {
+#pragma unroll
+        for (int o = 0; o < OCF; o++)
+#pragma unroll
+          for (int n = 0; n < PN; n++) tot[o][n] += acc[0][o][n];
+      };
+      constexpr std::true_type first{};
+      constexpr std::false_type next{};
+      int tt = 0;
+      if constexpr (MODE == kModeF16) {
+        while (tt < nt) {
+          const int end = min(tt + 9, nt);
+          tap(tt++, acc[0], first);
+          if (tt < end) {
+            tap(tt++, acc[1], first);
+            for (; tt + 2 <= end; tt += 2) {
+              tap(tt, acc[0], next);
+              tap(tt + 1, acc[1], next);
+            }
+            if (tt < end) tap(tt++, acc[0], next);
+#pragma unroll
+            for (int o = 0; o < OCF; o++)
+#pragma unroll
+              for (int n = 0; n < PN; n++) acc[0][o][n] += acc[1][o][n];
+          }
+          add_run();
+        }
+      } else {
+        for (; tt + 3 <= nt; tt += 3) {
+          tap(tt, acc[0], first);
+          tap(tt + 1, acc[0], next);
+          tap(tt + 2, acc[0], next);
+          add_run();
+        }
+        if (tt < nt) {
+          tap(tt, acc[0], first);
+          if (tt + 1 < nt) tap(tt + 1, acc[0], next);
+          add_run();
+        }
       }
       __syncthreads();  // the reads are done before the next copies, or the pool's stage, overwrite them
     }
-    if constexpr (BLOCKS) {
-#pragma unroll
-      for (int o = 0; o < OCF; o++)
-#pragma unroll
-        for (int n = 0; n < PN; n++) {
-          tot[o][n] += __builtin_bit_cast(v4f, acc[o][n]);
-          acc[o][n] = cb + 1 < s.blocks_c ? v4i{0, 0, 0, 0} : __builtin_bit_cast(v4i, tot[o][n]);
-        }
-    }
   }
-#define RG_CMF(ACTV) conv_mfma_out<MODE, ACTV, OCF, PN>(smem, acc, s, ep, b, oy0, ox0, o0, wave, lane)
+#define RG_CMF(ACTV) conv_mfma_out<MODE, ACTV, OCF, PN>(smem, tot, s, ep, b, oy0, ox0, o0, wave, lane)
   switch (ep.act) {
     case rgmath::ACT_RELU: RG_CMF(rgmath::ACT_RELU); break;
     case rgmath::ACT_SIGMOID: RG_CMF(rgmath::ACT_SIGMOID); break;

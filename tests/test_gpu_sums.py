@@ -69,3 +69,26 @@ def test_linear(rg, precision, rows, k, n):
         limit = _limit(64, k / 4 / 2 / 64)
     print(f"[sums lin] {precision} {rows}x{k}x{n} {e / U:.2f} u limit {limit / U:.2f} u", flush=True)
     assert e <= limit
+
+
+@pytest.mark.parametrize("precision", ["f32", "f16"])
+@pytest.mark.parametrize("images", [20, 3000])
+@pytest.mark.parametrize("c,o,k", [(32, 64, 3), (60, 64, 3), (128, 40, 3), (16, 64, 5), (64, 33, 5), (64, 64, 7),
+                                   (16, 40, 7), (256, 64, 1), (256, 96, 3)])
+def test_conv(rg, precision, c, o, k, images):
+    from rustgears_amd.inference import LayerSpec
+    rng = np.random.default_rng(c + o + k)
+    sums = []
+    for _ in range(6):
+        x = _values(rng, precision, (c, k, k), 6e4 / (c * k * k) ** 0.5)
+        w = _values(rng, precision, (o, c * k * k), 1.0)
+        sums.append(_error(rg, lambda b: LayerSpec.Conv2d(c, o, k, 1, 0, w.reshape(o, c, k, k), b), x, w,
+                           (images, c, k, k), precision))
+    e = np.sqrt(np.mean([a for a, _ in sums]) / np.mean([b for _, b in sums]))
+    # FP32: runs of three taps of 16 products; FP16: of nine taps, every other one, 32 products 8 at a time
+    if precision == "f32":
+        limit = _limit(48, -(-c // 16) * -(-k * k // 3))
+    else:
+        limit = _limit(5 * 4, 2 * -(-c // 32) * -(-k * k // 9))
+    print(f"[sums conv] {precision} conv {c}->{o} k {k} {images} images {e / U:.2f} u limit {limit / U:.2f} u", flush=True)
+    assert e <= limit
