@@ -246,6 +246,11 @@ __global__ __launch_bounds__(cmf::kThreads, 2) void conv_mfma_kernel(const float
           tap(tt++, acc[0], first);
           if (tt < end) {
             tap(tt++, acc[1], first);
+            if (end - tt == 7) {  // without branches, the reads run ahead of the MFMAs
+#pragma unroll
+              for (int u = 0; u < 7; u++) tap(tt + u, acc[u & 1], next);
+              tt = end;
+            }
             for (; tt + 2 <= end; tt += 2) {
               tap(tt, acc[0], next);
               tap(tt + 1, acc[1], next);
@@ -289,8 +294,19 @@ __global__ __launch_bounds__(cmf::kThreads, 2) void conv_mfma_kernel(const float
 
 // The tile of a convolution: whole output rows where they are at most 64
 // pixels wide, as many of them as 64, 128 or 256 pixels hold.  The largest of
-// those that still gives 1.5 workgroups per CU, else the smallest that fits
-// (the CNN's second conv on 100 images: 400 workgroups of 4 rows).
+// those that still gives 1.5 workgroups per CU, else the smallest that fits (the
+// CNN's second conv on 100 images: 400 workgroups of 4 rows); none that a smaller
+// one holds as well, whose pixels past the image would be multiplied for nothing
+// (256 images of 7 x 7, 256 -> 256: FP32 610 -> 194 us, FP16 117 -> 76 us), and not
+// 256 where 128 take far fewer rounds of the workgroups that a CU holds (100 images
+// of 23 x 23, 60 -> 120: FP32 132 -> 109 us, FP16 47 -> 35; 256 of 28 x 28, 128 -> 256,
+// 1 x 1: 276 -> 196 and 277 -> 154; but 256 of 14 x 14, 128 -> 128, one round of 256:
+// FP16 42 against 59; a window of 1 is mostly band, which more workgroups load
+// sooner).  Then fewer output channels while that gives at most two
+// workgroups per CU and the band is small: a workgroup walks all of K, and a short
+// walk is worth reading the band again (4 images of 14 x 14, 128 -> 128 channels: 64,
+// 32 and 16 of them FP32 33, 22 and 17 us, FP16 16, 14 and 10; but 7 x 7 at stride 2
+// on 1 x 3 x 224 x 224 FP16 25 and 37 us).
 struct ConvMfmaTile {
   int ocf = 0, pn = 0;
   ConvMfmaShape s{};
@@ -307,22 +323,35 @@ static bool conv_mfma_tile(const ConvShape& cs, bool f16, bool pool, ConvMfmaTil
   if (cs.n <= 0 || cs.OH <= 0 || cs.OW <= 0 || (pool && (cs.OH < 2 || cs.OW < 2)) ||
       cs.C * cs.H * cs.W * 4 >= (int64_t(1) << 31) || cs.k > 64)
     return false;
-  const int ocf = cs.O <= 16 ? 1 : cs.O <= 32 ? 2 : 4;
-  const int64_t XB = std::min<int64_t>(cs.OW, 64), ob = 16 * ocf;
-  const int64_t TG = std::max<int64_t>(1, std::min<int64_t>(cs.k * cs.k, cmf::kGroupBytes / (ob * 64)));
-  for (int pn : {4, 2, 1}) {
-    int64_t RB = std::min<int64_t>(cs.OH, 64 * pn / XB);
-    if (pool) RB &= ~int64_t(1);
-    if (RB <= 0) continue;
+  int ocf = cs.O <= 16 ? 1 : cs.O <= 32 ? 2 : 4;
+  const int64_t XB = std::min<int64_t>(cs.OW, 64);
+  auto rows = [&](int pn) {
+    const int64_t r = std::min<int64_t>(cs.OH, 64 * pn / XB);
+    return pool ? r & ~int64_t(1) : r;
+  };
+  auto tiles = [&](int pn) { return cs.n * ((cs.OH + rows(pn) - 1) / rows(pn)) * ((cs.OW + XB - 1) / XB); };
+  // 256 pixels leave a CU two workgroups, 128 three
+  const int64_t to = (cs.O + 63) / 64;
+  const bool half = rows(2) > 0 && rows(2) < rows(4) &&
+                    5 * ((tiles(2) * to + 767) / 768) < (cs.k == 1 ? 8 : 7) * ((tiles(4) * to + 511) / 512);
+  for (int pn = half ? 2 : 4; pn >= 1;) {
+    const int64_t RB = rows(pn), ob = 16 * ocf;
+    const int smaller = pn > 1 && rows(pn / 2) > 0 ? pn / 2 : 0;
+    if (RB <= 0 || (smaller >= 1 && rows(smaller) == RB)) {
+      pn = smaller;
+      continue;
+    }
+    const int64_t TG = std::max<int64_t>(1, std::min<int64_t>(cs.k * cs.k, cmf::kGroupBytes / (ob * 64)));
     const int64_t BR = (RB - 1) * cs.stride + cs.k, BC = (XB - 1) * cs.stride + cs.k;
     const int64_t band = (BR * BC * 64 + 1023) / 1024 * 1024;
-    // quotients by multiplication are exact while dividend * divisor < 2^32
-    if (4 * BR * BC >= 65536 || BC >= 65536 || BR >= 65536) continue;
     const int64_t lds = std::max(band + TG * ob * 64, pool ? ob * (64 * pn + 4) * 4 : int64_t(0));
-    if (lds > cmf::kMaxLds) continue;
     const int64_t ty = (cs.OH + RB - 1) / RB, tx = (cs.OW + XB - 1) / XB, to = (cs.O + ob - 1) / ob;
     const int64_t grid = cs.n * ty * tx * to;
-    if (grid >= (int64_t(1) << 31)) continue;
+    // quotients by multiplication are exact while dividend * divisor < 2^32
+    if (4 * BR * BC >= 65536 || BC >= 65536 || BR >= 65536 || lds > cmf::kMaxLds || grid >= (int64_t(1) << 31)) {
+      pn = smaller;
+      continue;
+    }
     ConvMfmaTile g;
     g.ocf = ocf;
     g.pn = pn;
@@ -346,6 +375,12 @@ static bool conv_mfma_tile(const ConvShape& cs, bool f16, bool pool, ConvMfmaTil
     s.wbase = (int32_t)band;
     *out = g;
     if (grid >= 384) break;
+    if (smaller >= 1)
+      pn = smaller;
+    else if (ocf > 1 && 4 * BR * BC <= 2048 && cs.n * ty * tx * ((cs.O + ob / 2 - 1) / (ob / 2)) <= 512)
+      ocf /= 2;
+    else
+      break;
   }
   return out->ocf != 0;
 }
@@ -353,6 +388,17 @@ static bool conv_mfma_tile(const ConvShape& cs, bool f16, bool pool, ConvMfmaTil
 bool conv_mfma_supported(const ConvShape& cs, bool f16, bool pool) {
   ConvMfmaTile g;
   return conv_mfma_tile(cs, f16, pool, &g);
+}
+
+// A workgroup walks all of K (a tap of a channel block ~0.1 us, the next block's
+// band ~1.2), where im2col + GEMM splits it over the chip for four launches: deep
+// layers on few pixels are faster there (3 x 3 on 7 x 7 images, 512 -> 512 channels,
+// one image: FP32 65 against 49 us, FP16 38 against 32; 256 -> 256 FP32 38 against
+// 32, but on 16 images 40 against 51).
+bool conv_mfma_better(const ConvShape& cs, bool f16) {
+  const int64_t per = f16 ? 32 : 16, blocks = (cs.C + per - 1) / per, walk = blocks * (cs.k * cs.k + 12);
+  const int64_t pixels = cs.n * cs.OH * cs.OW;
+  return f16 ? walk < 160 || pixels > 4 * (walk - 110) : walk < 320 || pixels > 2 * (walk - 200);
 }
 
 template <int MODE, int OCF, int PN>

@@ -861,8 +861,10 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
         for (auto v : rm) pl.full_cov &= v != 0;
         for (auto v : cm) pl.full_cov &= v != 0;
         if (P->precision != RGNPU_PRECISION_INT8 && pl.rows > 0 && !conv_direct(op)) {
-          const char* e = getenv("RGNPU_CONV_MFMA");  // 0: im2col + GEMM (tests, measurements)
-          pl.cmf = !(e && atoi(e) == 0) && conv_mfma_supported(pl.cs, P->precision == RGNPU_PRECISION_FP16, false);
+          const bool f16 = P->precision == RGNPU_PRECISION_FP16;
+          const char* e = getenv("RGNPU_CONV_MFMA");  // 0: im2col + GEMM, 2: this kernel (tests, measurements)
+          const int mode = e ? atoi(e) : 1;
+          pl.cmf = mode != 0 && (mode == 2 || conv_mfma_better(pl.cs, f16)) && conv_mfma_supported(pl.cs, f16, false);
         }
         pl.mask_off = (int64_t)mask_host.size();
         mask_host.insert(mask_host.end(), rm.begin(), rm.end());

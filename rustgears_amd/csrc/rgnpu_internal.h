@@ -350,6 +350,7 @@ void launch_conv_direct_f32(const float* x, const float* w, const float* bias, f
 // one per image).
 constexpr int64_t kConvMfmaOPad = 64;
 bool conv_mfma_supported(const ConvShape& cs, bool f16, bool pool);
+bool conv_mfma_better(const ConvShape& cs, bool f16);  // than im2col + GEMM
 void launch_conv_mfma(const float* x, const void* w, const ConvShape& cs, bool f16, bool pool, const Epilogue& ep,
                       hipStream_t s);
 void load_conv_mfma_code_object(hipStream_t s);
