@@ -1043,6 +1043,21 @@ int64_t gemm_workspace_bytes(int64_t Mpad, int64_t Npad, int64_t Kpad) {
   return g.splits > 1 ? (int64_t)g.splits * Mpad * Npad * 4 : 0;
 }
 
+// FP32: the matrix cores take 1.0 us per K step (64 bytes of each row) of a 128 x
+// 128 tile and 5 us around it, a tile per CU and round; split sums go through
+// memory and a second kernel (us: 777 x 4096 x 4096 estimated 265, measured 272;
+// 200 x 4096 x 4096, K in 8 slices, 84 and 82; 1300 x 1024 x 8192 211 and 211).
+double gemm_f32_us(int64_t M, int64_t Mpad, int64_t Npad, int64_t Kpad_bytes) {
+  const GemmChoice g = choose_gemm(M, Mpad, Npad, Kpad_bytes);
+  const int64_t nk = Kpad_bytes / big::BK;
+  if (g.splits > 1) {
+    const int64_t rounds = ((Mpad / 128) * (Npad / 128) * g.splits + 255) / 256;
+    return 7.0 + (double)(rounds * ((nk + g.splits - 1) / g.splits)) + (double)(g.splits * Mpad * Npad) * 8.0 / 5e6;
+  }
+  const int64_t rounds = ((M + g.bm - 1) / g.bm * (Npad / g.bn) + 255) / 256;
+  return 4.0 + (double)rounds * (double)(g.bm * g.bn) / 16384.0 * (double)(nk + 5);
+}
+
 template <int MODE>
 static void launch_gemm_t(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t Mpad, int64_t Npad,
                           int64_t Kpad, const Epilogue& ep, int32_t* ws, int64_t ws_bytes, hipStream_t s) {

@@ -324,11 +324,16 @@ static int64_t mid_rounds(const MidTile& t, int64_t M, int64_t N) {
 }
 
 // The tile with the least estimated time: a CU's K blocks at 40 bytes a clock
-// of loads or one MFMA every 16 clocks per SIMD (FP32: 128), whichever is
-// more, over the rounds of one workgroup per CU, plus 1 us a round and 2.5 us a
-// launch.  Over 27 shapes (9 to 2000 rows, each precision) the tile it takes
-// was the fastest of the nine or within 6% of it.  RGNPU_MID_TILE (an index,
-// for tests and measurements) forces a tile.
+// of loads or one MFMA every 16 clocks per SIMD, whichever is more, over the
+// rounds of one workgroup per CU, plus 1 us a round and 2.5 us a launch.  FP32
+// takes an MFMA's 32 clocks and the loads one after the other, and its rounds end
+// with more partial sums to write (4096 x 4096, us per round, estimated and
+// measured: 16 x 16 10.0 and 10.2, 32 x 32 26 and 26, 64 x 64 79 and 81, 128 x 64
+// 147 and 146).  Over 27 shapes (9 to 2000 rows, each precision) the tile it takes
+// was the fastest of the nine or within 6% of it; of 87 FP32 shapes (200 to 8192
+// rows) it and gemm_f32_us together took the fastest kernel or one within 1% on
+// average, 14% at most.  RGNPU_MID_TILE (an index, for tests and measurements)
+// forces a tile.
 int mid_choice(int mode, int64_t M, int64_t N, int64_t kb, double* us) {
   int best = 0;
   double best_us = 0.0;
@@ -337,7 +342,8 @@ int mid_choice(int mode, int64_t M, int64_t N, int64_t kb, double* us) {
     const double rounds = (double)mid_rounds(t, M, N), steps = (double)(kb / 64);
     const double load = steps * (t.tm + t.tn) * 64.0 / 40.0;
     const double mfma = steps * (t.tm / 16) * (t.tn / 16) * (mode == kModeF32 ? 128.0 : 16.0) / 4.0;
-    const double c = 2.5 + rounds * (1.0 + (load > mfma ? load : mfma) / 2400.0);
+    const double work = mode == kModeF32 ? load + mfma + t.tm * t.tn : load > mfma ? load : mfma;
+    const double c = 2.5 + rounds * (1.0 + work / 2400.0);
     if (i == 0 || c < best_us) {
       best = i;
       best_us = c;
@@ -346,20 +352,6 @@ int mid_choice(int mode, int64_t M, int64_t N, int64_t kb, double* us) {
   if (us) *us = best_us;
   if (const char* e = getenv("RGNPU_MID_TILE")) best = std::min(kMidTileCount - 1, std::max(0, atoi(e)));
   return best;
-}
-
-// FP32 is bound by the matrix cores, so the tiles that leave the busiest CU
-// the fewest outputs win; the tile GEMM's rate per output is 13% better (1000 x
-// 4096 x 4096: 257 against 290 us), its 128 x 128 and larger tiles divide
-// worse over the CUs (3000 x 4096 x 4096, 384 tiles of 256 x 128: 942 against
-// 873 us; 300 x 4096 x 4096: 252 against 132 us).
-bool mid_f32_better(int64_t M, int64_t N, int64_t big_tiles, int64_t big_area) {
-  double mid = 0.0;
-  for (const MidTile& t : kMidTiles) {
-    const double u = (double)(mid_rounds(t, M, N) * t.tm * t.tn);
-    if (mid == 0.0 || u < mid) mid = u;
-  }
-  return 1.13 * mid < (double)((big_tiles + 255) / 256 * big_area);
 }
 
 bool gemm_mid_supported(int64_t M, int64_t N, int64_t lda, int64_t kb) {

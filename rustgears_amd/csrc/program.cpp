@@ -785,7 +785,10 @@ static int conv_pool_fusion(const rgnpu_program* P, const std::vector<OpPlan>& p
 //    takes what this one and the quantize pass take (2048 x 384 x 512: 8.6
 //    against 4.8 + 3.7 us).
 //  * INT8 heads of at most 16 outputs quantize as they read (launch_gemm_narrow).
-//  * FP32 is bound by the matrix cores (mid_f32_better).
+//  * FP32 is bound by the matrix cores, so tiles that divide well over the CUs
+//    count for more than loads: both kernels' times are estimated (777 x 4096 x
+//    4096: 272 us as 224 tiles of 128 x 128, 308 and more here; 400 x 4096 x 4096
+//    260 and 157; 400 x 8192 x 1024 82 and 92).
 //  * FP16 and FP32 on 2 to 8 rows with 16 MB of weights or more, where the
 //    streamed weights go through LDS here and each activation row costs the
 //    GEMV another load per weight load (5 x 14336 x 4096: FP16 37.3 -> 17.6 us,
@@ -803,14 +806,20 @@ static bool use_mid(const rgnpu_program* P, const Op& op, const OpPlan& pl) {
     return P->precision != RGNPU_PRECISION_INT8 && pl.rows > 1 &&
            (mode == 2 || op.out_f * op.Kpad * es >= (int64_t(16) << 20));
   if (mode != 1) return mode == 2;
+  if (P->precision == RGNPU_PRECISION_FP32) {
+    if (op.out_f <= kNarrowMaxN) return true;
+    double us = 0.0;
+    mid_choice(2, pl.rows, op.out_f, op.Kpad * es, &us);
+    // the tile GEMM reads whole padded rows, this one the input itself
+    const bool pads = pl.rows != pl.Mpad || op.K != op.Kpad;
+    const double pad_us = pads ? 3.0 + 2e-6 * (double)(pl.rows * op.K) : 0.0;
+    return us <= gemm_f32_us(pl.rows, pl.Mpad, op.Npad, op.Kpad * es) + pad_us;
+  }
   const int64_t tiles = ((pl.rows + 127) / 128) * ((op.out_f + 127) / 128);
   const GemmChoice g = choose_gemm(pl.rows, pl.Mpad, op.Npad, op.Kpad * es);
   if (P->precision == RGNPU_PRECISION_INT8)
     return op.out_f > kNarrowMaxN && (tiles < 48 || (tiles < 128 && g.splits > 1));
-  if (op.out_f <= kNarrowMaxN || g.splits > 1) return true;
-  if (P->precision == RGNPU_PRECISION_FP16) return tiles <= 128;
-  return mid_f32_better(pl.rows, op.out_f, ((pl.rows + g.bm - 1) / g.bm) * ((op.out_f + g.bn - 1) / g.bn),
-                        (int64_t)g.bm * g.bn);
+  return op.out_f <= kNarrowMaxN || g.splits > 1 || tiles <= 128;
 }
 
 // With `scratch` the plan's buffers are views into that device array (of

@@ -160,6 +160,7 @@ struct GemmChoice {
   int splits;
 };
 GemmChoice choose_gemm(int64_t M, int64_t Mpad, int64_t Npad, int64_t Kpad);
+double gemm_f32_us(int64_t M, int64_t Mpad, int64_t Npad, int64_t Kpad_bytes);  // estimated time of launch_gemm_f32
 
 // The same GEMM with the next Linear's quantization fused (requant.hip):
 // a persistent grid computes every tile and its fused epilogue, raises
@@ -193,7 +194,6 @@ void launch_input_quant(const float* x, int64_t M, int64_t K, int64_t Mpad, int6
 // mid_choice: the tile (an index) with the least estimated time, in us.
 bool gemm_mid_supported(int64_t M, int64_t N, int64_t lda_bytes, int64_t kb_bytes);
 int mid_choice(int mode, int64_t M, int64_t N, int64_t kb_bytes, double* us);
-bool mid_f32_better(int64_t M, int64_t N, int64_t big_tiles, int64_t big_area);
 void launch_gemm_mid(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t Kpad, const Epilogue& ep,
                      hipStream_t s);
 void launch_gemm_mid_f16(const uint16_t* A, const uint16_t* B, int64_t M, int64_t N, int64_t Kpad_h,
