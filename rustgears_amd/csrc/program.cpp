@@ -818,7 +818,8 @@ static bool use_mid(const rgnpu_program* P, const Op& op, const OpPlan& pl) {
   const int64_t tiles = ((pl.rows + 127) / 128) * ((op.out_f + 127) / 128);
   const GemmChoice g = choose_gemm(pl.rows, pl.Mpad, op.Npad, op.Kpad * es);
   if (P->precision == RGNPU_PRECISION_INT8)
-    return op.out_f > kNarrowMaxN && (tiles < 48 || (tiles < 128 && g.splits > 1));
+    return op.out_f > kNarrowMaxN &&
+           (tiles < 48 || (tiles < 128 && g.splits > 1));
   return op.out_f <= kNarrowMaxN || g.splits > 1 || tiles <= 128;
 }
 

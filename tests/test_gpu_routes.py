@@ -17,7 +17,7 @@ def _run(rg, monkeypatch, layers, x, mid):
 
 
 @pytest.mark.parametrize("rows,k,n,small_tiles", [(777, 4096, 4096, False), (1300, 1024, 8192, False),
-                                                  (1300, 4096, 4096, False), (400, 4096, 4096, True),
+                                                  (1300, 4096, 4096, True), (400, 4096, 4096, True),
                                                   (1000, 1024, 1024, True), (2000, 1024, 1024, True)])
 def test_fp32_small_tiles_or_large(rg, monkeypatch, rows, k, n, small_tiles):
     """FP32 on the small-tile GEMM only where it is the faster one; the two sum
