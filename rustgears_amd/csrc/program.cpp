@@ -780,10 +780,13 @@ static int conv_pool_fusion(const rgnpu_program* P, const std::vector<OpPlan>& p
 // 128 x 128 those leave CUs idle or split K (1000 x 1024 x 1024 i8: 17.6
 // against 5.8 us; above, the larger tiles load less: 1000 x 4096 x 4096 i8
 // 24.9 against 29.5 us, f16 44.4 against 51.2 us).  Exceptions:
-//  * INT8 from 48 tiles on, K not split (up to 7 K steps of 64): the tile GEMM
-//    also quantizes its outputs for the next Linear, and one kernel of it
-//    takes what this one and the quantize pass take (2048 x 384 x 512: 8.6
-//    against 4.8 + 3.7 us).
+//  * INT8 from 48 tiles on with up to 7 K steps of 64: the tile GEMM also
+//    quantizes its outputs for the next Linear, and one kernel of it takes what
+//    this one and the quantize pass take (2048 x 384 x 512: 8.6 against 4.8 + 3.7
+//    us).  Up to 128 rows have half of the tiles that their padded 256 would (12 x
+//    14336 x 8192: 62 against 18.5 us); there it holds from 96 tiles on also for
+//    more than 64 rows and K below 4096 (100 x 1024 x 14000 GELU and the next layer
+//    29.7 against 32.3 us; 33 rows 27.8 and 22.2, K 8192 56 and 49).
 //  * INT8 heads of at most 16 outputs quantize as they read (launch_gemm_narrow).
 //  * FP32 is bound by the matrix cores, so tiles that divide well over the CUs
 //    count for more than loads: both kernels' times are estimated (777 x 4096 x
@@ -819,7 +822,9 @@ static bool use_mid(const rgnpu_program* P, const Op& op, const OpPlan& pl) {
   const GemmChoice g = choose_gemm(pl.rows, pl.Mpad, op.Npad, op.Kpad * es);
   if (P->precision == RGNPU_PRECISION_INT8)
     return op.out_f > kNarrowMaxN &&
-           (tiles < 48 || (tiles < 128 && g.splits > 1));
+           (tiles < 48 || (tiles < 128 && (pl.rows > 128 ? g.splits > 1
+                                                         : op.Kpad >= 512 && (tiles < 96 || pl.rows <= 64 ||
+                                                                              op.Kpad >= 4096))));
   return op.out_f <= kNarrowMaxN || g.splits > 1 || tiles <= 128;
 }
 

@@ -29,3 +29,23 @@ def test_fp32_small_tiles_or_large(rg, monkeypatch, rows, k, n, small_tiles):
     y, large, small = (_run(rg, monkeypatch, layers, x, mid) for mid in (None, "0", "2"))
     assert not np.array_equal(large, small)
     assert np.array_equal(y, small if small_tiles else large)
+
+
+@pytest.mark.parametrize("rows,k,n,small_tiles", [(9, 1024, 8192, True), (128, 512, 8192, True), (12, 512, 14000, True),
+                                                  (128, 512, 14000, False), (9, 384, 8192, False),
+                                                  (300, 512, 4096, False)])
+def test_int8_up_to_128_rows(rg, ref, monkeypatch, rows, k, n, small_tiles):
+    """An INT8 Linear on up to 128 rows has half of the tiles of its padded 256;
+    on the small-tile GEMM the next Linear quantizes its input in a pass of its
+    own, on the tile GEMM it comes quantized."""
+    from conftest import assert_bitexact_f32
+    from rustgears_amd import nn
+    monkeypatch.setenv("RGNPU_SMALL_XQ", "0")  # which would quantize as it reads
+    rg.manual_seed(rows + n)
+    layers = nn.Sequential().add(nn.Linear(k, n)).add(nn.Relu()).add(nn.Linear(n, 40)).export()
+    x = rg.randn([rows, k])
+    sess = rg.InferenceSession.from_layers(layers, rg.ExecutionProvider.mi355x_int8())
+    assert_bitexact_f32(sess.run(x), ref.RefProgram(layers).run(x, parallel=True), f"{rows} {k} {n}")
+    second = sess.last_npu_profile().records[1]
+    sess.close()
+    assert (second.duration_ns > second.kernel_ns) == small_tiles, second
