@@ -4,6 +4,8 @@
 #include <hip/hip_runtime_api.h>
 #include <stdint.h>
 
+#include "gemm_choice.h"
+
 namespace rgnpu {
 
 // Padding rules for device operands.  Weights are stored [Npad, Kpad] with
@@ -152,15 +154,6 @@ void launch_gemm(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t
 // workspace of this many bytes (f32 partial sums); without one they run
 // unsplit.
 int64_t gemm_workspace_bytes(int64_t Mpad, int64_t Npad, int64_t Kpad);
-// Tile shape of the large GEMM: 256, 192 or 128 rows x 256 columns (8 waves), or
-// 128 x 128 (4 waves); splits > 1 when K is split.  The tiles of M rows cover no
-// more than Mpad.
-struct GemmChoice {
-  int bm, bn;
-  int splits;
-};
-GemmChoice choose_gemm(int64_t M, int64_t Mpad, int64_t Npad, int64_t Kpad);
-double gemm_f32_us(int64_t M, int64_t Mpad, int64_t Npad, int64_t Kpad_bytes);  // estimated time of launch_gemm_f32
 
 // The same GEMM with the next Linear's quantization fused (requant.hip):
 // a persistent grid computes every tile and its fused epilogue, raises
