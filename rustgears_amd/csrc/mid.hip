@@ -29,7 +29,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstdlib>
 #include <stdexcept>
 #include <type_traits>
 
@@ -315,7 +314,7 @@ struct MidTile {
 };
 static constexpr MidTile kMidTiles[] = {{16, 16}, {16, 32}, {16, 64}, {32, 32}, {64, 32},
                                         {32, 64}, {64, 64}, {128, 64}, {64, 128}};
-static constexpr int kMidTileCount = (int)(sizeof kMidTiles / sizeof kMidTiles[0]);
+static_assert(sizeof kMidTiles / sizeof kMidTiles[0] == kMidTileCount, "tile indexes");
 
 // Rounds of one workgroup on each of the 256 CUs (a workgroup's LDS leaves
 // room for no second one).
@@ -332,8 +331,7 @@ static int64_t mid_rounds(const MidTile& t, int64_t M, int64_t N) {
 // 147 and 146).  Over 27 shapes (9 to 2000 rows, each precision) the tile it takes
 // was the fastest of the nine or within 6% of it; of 87 FP32 shapes (200 to 8192
 // rows) it and gemm_f32_us together took the fastest kernel or one within 1% on
-// average, 14% at most.  RGNPU_MID_TILE (an index, for tests and measurements)
-// forces a tile.
+// average, 14% at most.
 int mid_choice(int mode, int64_t M, int64_t N, int64_t kb, double* us) {
   int best = 0;
   double best_us = 0.0;
@@ -350,7 +348,6 @@ int mid_choice(int mode, int64_t M, int64_t N, int64_t kb, double* us) {
     }
   }
   if (us) *us = best_us;
-  if (const char* e = getenv("RGNPU_MID_TILE")) best = std::min(kMidTileCount - 1, std::max(0, atoi(e)));
   return best;
 }
 
@@ -376,14 +373,14 @@ static void launch_mid_t(const int8_t* A, const int8_t* B, MidShape s, const Epi
 
 template <int MODE>
 static void launch_mid_mode(const int8_t* A, int64_t lda, int64_t ka, const int8_t* B, int64_t M, int64_t N, int64_t kb,
-                            const Epilogue& ep, hipStream_t st) {
+                            int tile, const Epilogue& ep, hipStream_t st) {
   if (!gemm_mid_supported(M, N, lda, kb) || ka > kb || ka % 16 || (reinterpret_cast<uintptr_t>(A) & 15))
     throw std::logic_error("mid GEMM: unsupported shape or unaligned operand");
   if (ep.h_out && (ep.ldh % 4 || MODE != kModeF16)) throw std::logic_error("mid GEMM: operand hand-off is FP16 only");
   const MidShape s{lda,        (int32_t)ka, (int32_t)kb, (int32_t)M,
                    (int32_t)N, 0,           0,           N % 4 == 0 && (reinterpret_cast<uintptr_t>(ep.y) & 15) == 0,
                    1};
-  switch (mid_choice(MODE, M, N, kb, nullptr)) {
+  switch (tile) {
     case 0: launch_mid_t<MODE, 1, 1, 8, 6>(A, B, s, ep, st); break;
     case 1: launch_mid_t<MODE, 1, 2, 8, 5>(A, B, s, ep, st); break;
     case 2: launch_mid_t<MODE, 1, 4, 8, 3>(A, B, s, ep, st); break;
@@ -396,22 +393,22 @@ static void launch_mid_mode(const int8_t* A, int64_t lda, int64_t ka, const int8
   }
 }
 
-void launch_gemm_mid(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t Kpad, const Epilogue& ep,
-                     hipStream_t s) {
+void launch_gemm_mid(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t Kpad, int tile,
+                     const Epilogue& ep, hipStream_t s) {
   if (!ep.absmax_in) throw std::logic_error("mid GEMM: no absmax slot");
-  launch_mid_mode<kModeI8>(A, Kpad, Kpad, B, M, N, Kpad, ep, s);
+  launch_mid_mode<kModeI8>(A, Kpad, Kpad, B, M, N, Kpad, tile, ep, s);
 }
 
 void launch_gemm_mid_f16(const uint16_t* A, const uint16_t* B, int64_t M, int64_t N, int64_t Kpad_h,
-                         const Epilogue& ep, hipStream_t s) {
+                         int tile, const Epilogue& ep, hipStream_t s) {
   launch_mid_mode<kModeF16>(reinterpret_cast<const int8_t*>(A), 2 * Kpad_h, 2 * Kpad_h,
-                            reinterpret_cast<const int8_t*>(B), M, N, 2 * Kpad_h, ep, s);
+                            reinterpret_cast<const int8_t*>(B), M, N, 2 * Kpad_h, tile, ep, s);
 }
 
 void launch_gemm_mid_f32(const float* A, int64_t lda, int64_t K, const float* B, int64_t M, int64_t N, int64_t Kpad_f,
-                         const Epilogue& ep, hipStream_t s) {
+                         int tile, const Epilogue& ep, hipStream_t s) {
   launch_mid_mode<kModeF32>(reinterpret_cast<const int8_t*>(A), 4 * lda, 4 * K, reinterpret_cast<const int8_t*>(B), M,
-                            N, 4 * Kpad_f, ep, s);
+                            N, 4 * Kpad_f, tile, ep, s);
 }
 
 // This translation unit's code object, loaded at program creation.

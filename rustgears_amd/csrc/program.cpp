@@ -149,6 +149,7 @@ struct OpPlan {
   // kernel pair.
   int64_t iq_sync_base = -1;
   bool mid = false;  // Linear on the small-tile GEMM of mid.hip
+  int mid_tile = 0;  // its tile (mid_choice)
   bool cmf = false;  // FP16 / FP32 conv in one kernel (conv_mfma.hip)
   // FP32 Linear or such a conv -> Act: its epilogue applies the activation
   // (fused_act on it; act_fused on the Act op, which launches nothing).
@@ -961,6 +962,12 @@ static std::unique_ptr<Plan> make_plan(rgnpu_program* P, const int64_t* shape, i
     OpPlan& pl = plan->ops[i];
     if (op.kind != OP_LINEAR && op.kind != OP_CONV) continue;
     pl.mid = use_mid(P, op, pl);
+    if (pl.mid) {
+      const int mode = P->precision == RGNPU_PRECISION_INT8 ? 0 : P->precision == RGNPU_PRECISION_FP16 ? 1 : 2;
+      pl.mid_tile = mid_choice(mode, pl.rows, op.out_f, op.Kpad * (int64_t(1) << mode), nullptr);
+      const char* te = getenv("RGNPU_MID_TILE");  // an index (tests, measurements)
+      if (te) pl.mid_tile = std::min(kMidTileCount - 1, std::max(0, atoi(te)));
+    }
     if (P->precision != RGNPU_PRECISION_INT8) {
       // No activation quantization: binary16 (FP16) or f32 (FP32) operands,
       // the split-K workspace, and the conv's [n*L, O] GEMM output.
@@ -1490,7 +1497,8 @@ static int enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEv
             ep.y_stream = pl.out_buf == BUF_OUTPUT;
             pre = launch_events_used();
             if (pl.mid)
-              launch_gemm_mid_f32(a, lda, lda, op.d_w.as<float>(), pl.rows, op.out_f, op.Kpad, ep, s);
+              launch_gemm_mid_f32(a, lda, lda, op.d_w.as<float>(), pl.rows, op.out_f, op.Kpad,
+                                  pl.mid_tile, ep, s);
             else if (pl.gemv)
               launch_gemv_f32(a, op.d_w.as<float>(), pl.rows, op.out_f, op.Npad, op.Kpad, ep, s);
             else
@@ -1523,7 +1531,7 @@ static int enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEv
             }
             pre = launch_events_used();
             if (pl.mid)
-              launch_gemm_mid_f16(h, op.d_w.as<uint16_t>(), pl.rows, op.out_f, op.Kpad, ep, s);
+              launch_gemm_mid_f16(h, op.d_w.as<uint16_t>(), pl.rows, op.out_f, op.Kpad, pl.mid_tile, ep, s);
             else if (pl.gemv)
               launch_gemv_f16(h, op.d_w.as<uint16_t>(), pl.rows, op.out_f, op.Npad, op.Kpad, ep, s);
             else
@@ -1598,7 +1606,7 @@ static int enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEv
             launch_gemm_narrow_xq(in, op.d_w.as<int8_t>(), pl.rows, op.out_f, op.in_f, op.Kpad, ep, cap ? qa : nullptr,
                                   cap ? scales + pl.scale_base : nullptr, s);
           } else if (pl.mid) {
-            launch_gemm_mid(qa, op.d_w.as<int8_t>(), pl.rows, op.out_f, op.Kpad, ep, s);
+            launch_gemm_mid(qa, op.d_w.as<int8_t>(), pl.rows, op.out_f, op.Kpad, pl.mid_tile, ep, s);
           } else if (op.out_f <= kNarrowMaxN) {
             launch_gemm_narrow(qa, op.d_w.as<int8_t>(), pl.rows, op.out_f, op.Kpad, ep, s);
           } else {

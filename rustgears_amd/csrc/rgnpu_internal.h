@@ -184,15 +184,17 @@ void launch_input_quant(const float* x, int64_t M, int64_t K, int64_t Mpad, int6
 // rows; Kpad is B's row length (zeros past K).  INT8 and FP16 read the padded
 // operand [>= M, Kpad]; FP32 reads the input itself: rows lda floats apart of
 // K floats (K and lda multiples of 4, 16-byte aligned base).
-// mid_choice: the tile (an index) with the least estimated time, in us.
+// mid_choice: the tile (an index below kMidTileCount) with the least estimated
+// time, in us; a plan keeps it for its launches.
+constexpr int kMidTileCount = 9;
 bool gemm_mid_supported(int64_t M, int64_t N, int64_t lda_bytes, int64_t kb_bytes);
 int mid_choice(int mode, int64_t M, int64_t N, int64_t kb_bytes, double* us);
-void launch_gemm_mid(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t Kpad, const Epilogue& ep,
-                     hipStream_t s);
+void launch_gemm_mid(const int8_t* A, const int8_t* B, int64_t M, int64_t N, int64_t Kpad, int tile,
+                     const Epilogue& ep, hipStream_t s);
 void launch_gemm_mid_f16(const uint16_t* A, const uint16_t* B, int64_t M, int64_t N, int64_t Kpad_h,
-                         const Epilogue& ep, hipStream_t s);
+                         int tile, const Epilogue& ep, hipStream_t s);
 void launch_gemm_mid_f32(const float* A, int64_t lda, int64_t K, const float* B, int64_t M, int64_t N, int64_t Kpad_f,
-                         const Epilogue& ep, hipStream_t s);
+                         int tile, const Epilogue& ep, hipStream_t s);
 void load_mid_code_object(hipStream_t s);
 
 // INT8 Linear with N <= kNarrowMaxN outputs per row: one wave per row, the

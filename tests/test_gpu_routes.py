@@ -49,3 +49,21 @@ def test_int8_up_to_128_rows(rg, ref, monkeypatch, rows, k, n, small_tiles):
     second = sess.last_npu_profile().records[1]
     sess.close()
     assert (second.duration_ns > second.kernel_ns) == small_tiles, second
+
+
+def test_the_tile_is_chosen_with_the_plan(rg, monkeypatch):
+    """The environment is read when a plan is made, not by each run: another
+    thread may be setting a variable then."""
+    from rustgears_amd.inference import LayerSpec
+    rg.manual_seed(3)
+    layers = [LayerSpec.Linear(3000, 200, rg.randn([600000]), rg.randn([200]))]
+    x = rg.randn([40, 3000])
+    sess = rg.InferenceSession.from_layers(layers, rg.ExecutionProvider.Gpu(0))
+    monkeypatch.setenv("RGNPU_MID_TILE", "0")
+    y = sess.run(x)
+    monkeypatch.setenv("RGNPU_MID_TILE", "6")  # sums over half as many slices of K
+    assert np.array_equal(sess.run(x), y)
+    other = rg.InferenceSession.from_layers(layers, rg.ExecutionProvider.Gpu(0))
+    assert not np.array_equal(other.run(x), y)
+    sess.close()
+    other.close()
