@@ -22,19 +22,21 @@ namespace rgnpu {
 // Launch-event sink (see set_launch_events): every kernel launched while it
 // is set carries the next event as the stop event of its own dispatch.
 static thread_local hipEvent_t* t_sink = nullptr;
-static thread_local int t_sink_cap = 0, t_sink_used = 0;
+static thread_local int t_sink_cap = 0, t_sink_used = 0, t_sink_only = kEveryLaunch;
 
-void set_launch_events(hipEvent_t* events, int cap) {
+void set_launch_events(hipEvent_t* events, int cap, int only) {
   t_sink = events;
   t_sink_cap = cap;
   t_sink_used = 0;
+  t_sink_only = only;
 }
 
 int launch_events_used() { return t_sink_used; }
 
 hipEvent_t next_launch_event() {
-  if (t_sink && t_sink_used < t_sink_cap) return t_sink[t_sink_used++];
-  return nullptr;
+  if (!t_sink || t_sink_used >= t_sink_cap) return nullptr;
+  const int i = t_sink_used++;
+  return t_sink_only == kEveryLaunch || t_sink_only == i ? t_sink[i] : nullptr;
 }
 
 // ---------------------------------------------------------------------------

@@ -219,6 +219,7 @@ struct Plan {
   // [0] last launch before the op, [1] last launch before its main kernel,
   // [2] its main kernel (== [1] when the op launches none).
   std::vector<std::array<int, 3>> roles;
+  int launches = 0;  // kernels of the last run
 };
 
 }  // namespace rgnpu
@@ -1397,7 +1398,9 @@ static void op_times(const Plan& plan, hipEvent_t start, const hipEvent_t* set, 
 // A null `ev` records nothing (back-to-back throughput runs).  Returns the
 // number of kernels launched.
 enum { MARK_START = 1, MARK_END = 2 };
-static int enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEvent_t* ev, int marks) {
+// With `only` just that launch records its event, and the plan has no roles.
+static int enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEvent_t* ev, int marks,
+                   int only = kEveryLaunch) {
   hipStream_t s = P->stream;
   const bool f16 = P->precision == RGNPU_PRECISION_FP16;
   const bool f32 = P->precision == RGNPU_PRECISION_FP32;
@@ -1408,7 +1411,7 @@ static int enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEv
   struct SinkOff {
     ~SinkOff() { set_launch_events(nullptr, 0); }
   } sink_off;
-  set_launch_events(ev ? ev + 2 : nullptr, ev ? (int)launch_event_cap(P) : 0);
+  set_launch_events(ev ? ev + 2 : nullptr, ev ? (int)launch_event_cap(P) : 0, only);
   if (cap) ensure_capture_buffers(P, plan);
   if (tap) ensure_tap_buffers(P, plan);
   plan.roles.assign(P->ops.size(), std::array<int, 3>{-1, -1, -1});
@@ -1828,7 +1831,7 @@ static int enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEv
                               hipMemcpyDeviceToDevice, s));
     }
     const int end = launch_events_used();
-    plan.roles[i] = {first - 1, pre - 1, end > pre ? end - 1 : pre - 1};
+    if (only == kEveryLaunch) plan.roles[i] = {first - 1, pre - 1, end > pre ? end - 1 : pre - 1};
   }
   const int launched = launch_events_used();
   if (ev && (size_t)launched >= launch_event_cap(P))
@@ -1850,9 +1853,11 @@ static int enqueue(rgnpu_program* P, Plan& plan, const float* x, float* y, hipEv
 // So the last kernel's event ends the run, and a device-resident run enqueued
 // while the previous one is still under way starts at that one's end: nothing
 // else is on the stream (should it end before this run's first kernel arrives,
-// that gap, less than the enqueue takes, is counted).  A run on an idle stream, after other work
-// (`after_work`: a host copy), with copies of its own (capture) or without
-// kernels keeps its markers.
+// that gap, less than the enqueue takes, is counted).  A run on an idle stream,
+// after other work (`after_work`: a host copy), with copies of its own (capture)
+// or without kernels keeps its markers.  With profiling off the last kernel
+// alone records its event (the plan's runs launch the same kernels; the first
+// run, or one that differs, ends in a marker).
 static void enqueue_profiled(rgnpu_program* P, Plan& plan, const float* x, float* y, bool after_work) {
   ensure_events(P);
   hipEvent_t* const set = P->ev.data() + (size_t)(P->ev_set ^= 1) * events_per_run(P);
@@ -1867,9 +1872,11 @@ static void enqueue_profiled(rgnpu_program* P, Plan& plan, const float* x, float
   P->last_event = nullptr;
   P->profile_pending = false;
   const bool copies = P->capture || P->taps;
-  const int launched = enqueue(P, plan, x, y, set, (mark ? MARK_START : 0) | (copies ? MARK_END : 0));
+  const int only = P->profiling > 0 ? kEveryLaunch : plan.launches > 0 ? plan.launches - 1 : kNoLaunch;
+  const int launched = enqueue(P, plan, x, y, set, (mark ? MARK_START : 0) | (copies ? MARK_END : 0), only);
+  plan.launches = launched;
   hipEvent_t end = set[1];
-  if (!copies && launched > 0)
+  if (!copies && launched > 0 && (only == kEveryLaunch || only == launched - 1))
     end = set[2 + launched - 1];
   else if (!copies)
     RG_HIP(hipEventRecord(end, P->stream));
@@ -1899,12 +1906,10 @@ static void finalize_profile(rgnpu_program* P) {
     snprintf(r.op, sizeof r.op, "%s", P->ops[i]->label.c_str());
     r.macs = plan.ops[i].macs;
     total_macs += r.macs;
-    if (P->profiling > 0) {
-      double a = 0, b = 0;
-      op_times(plan, P->prof_start, P->ev.data() + (size_t)P->ev_set * events_per_run(P), i, &a, &b);
-      r.ns = (uint64_t)(a * 1e6);
-      r.kernel_ns = (uint64_t)(b * 1e6);
-    }
+    double a = 0, b = 0;  // zero for a run with profiling off, which has no roles
+    op_times(plan, P->prof_start, P->ev.data() + (size_t)P->ev_set * events_per_run(P), i, &a, &b);
+    r.ns = (uint64_t)(a * 1e6);
+    r.kernel_ns = (uint64_t)(b * 1e6);
   }
   pr.total_macs = total_macs;
   pr.n_records = (int32_t)P->ops.size();

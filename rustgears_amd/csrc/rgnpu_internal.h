@@ -103,8 +103,10 @@ double probe_barrier_poll(uint32_t* lines, int blocks, int polls, hipStream_t s)
 // as the stop event of its own dispatch (hipExtLaunchKernelGGL), i.e. the
 // completion timestamp of that kernel, with no marker packet and no bubble
 // before the next kernel.  launch_events_used() counts the launches so far.
-// set_launch_events(nullptr, 0) turns it off.
-void set_launch_events(hipEvent_t* events, int cap);
+// With `only` the launch of that number alone records its event (kNoLaunch:
+// none do).  set_launch_events(nullptr, 0) turns it off.
+constexpr int kEveryLaunch = -1, kNoLaunch = -2;
+void set_launch_events(hipEvent_t* events, int cap, int only = kEveryLaunch);
 int launch_events_used();
 
 void launch_fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t s);
