@@ -325,11 +325,12 @@ static bool conv_mfma_tile(const ConvShape& cs, bool f16, bool pool, ConvMfmaTil
     return false;
   int ocf = cs.O <= 16 ? 1 : cs.O <= 32 ? 2 : 4;
   const int64_t XB = std::min<int64_t>(cs.OW, 64);
+  const int64_t used = pool ? cs.OH & ~int64_t(1) : cs.OH;  // the pool drops an odd last row
   auto rows = [&](int pn) {
-    const int64_t r = std::min<int64_t>(cs.OH, 64 * pn / XB);
+    const int64_t r = std::min<int64_t>(used, 64 * pn / XB);
     return pool ? r & ~int64_t(1) : r;
   };
-  auto tiles = [&](int pn) { return cs.n * ((cs.OH + rows(pn) - 1) / rows(pn)) * ((cs.OW + XB - 1) / XB); };
+  auto tiles = [&](int pn) { return cs.n * ((used + rows(pn) - 1) / rows(pn)) * ((cs.OW + XB - 1) / XB); };
   // 256 pixels leave a CU two workgroups, 128 three
   const int64_t to = (cs.O + 63) / 64;
   const bool half = rows(2) > 0 && rows(2) < rows(4) &&
@@ -345,7 +346,7 @@ static bool conv_mfma_tile(const ConvShape& cs, bool f16, bool pool, ConvMfmaTil
     const int64_t BR = (RB - 1) * cs.stride + cs.k, BC = (XB - 1) * cs.stride + cs.k;
     const int64_t band = (BR * BC * 64 + 1023) / 1024 * 1024;
     const int64_t lds = std::max(band + TG * ob * 64, pool ? ob * (64 * pn + 4) * 4 : int64_t(0));
-    const int64_t ty = (cs.OH + RB - 1) / RB, tx = (cs.OW + XB - 1) / XB, to = (cs.O + ob - 1) / ob;
+    const int64_t ty = (used + RB - 1) / RB, tx = (cs.OW + XB - 1) / XB, to = (cs.O + ob - 1) / ob;
     const int64_t grid = cs.n * ty * tx * to;
     // quotients by multiplication are exact while dividend * divisor < 2^32
     if (4 * BR * BC >= 65536 || BC >= 65536 || BR >= 65536 || lds > cmf::kMaxLds || grid >= (int64_t(1) << 31)) {

@@ -60,3 +60,19 @@ def test_deep_layers_on_few_pixels(rg, ref, n, c, hw, im2col):
     sess.close()
     # im2col runs before the op's main kernel
     assert (r.duration_ns > r.kernel_ns) == im2col, r
+
+
+@pytest.mark.parametrize("hw", [4, 6, 8, 11])
+def test_small_images_pool_in_the_convolution(rg, hw):
+    """Images of fewer than 128 pixels too: the pool launches nothing and the
+    Linear after it converts nothing."""
+    from rustgears_amd import nn
+    rg.manual_seed(hw)
+    layers = (nn.Sequential().add(nn.Conv2d(32, 64, 3).padding(1)).add(nn.Relu()).add(nn.MaxPool2d(2))
+              .add(nn.Flatten()).add(nn.Linear(64 * (hw // 2) ** 2, 64))).export()
+    sess = rg.InferenceSession.from_layers(layers, rg.ExecutionProvider.mi355x_fp16())
+    sess.run(rg.randn([20, 32, hw, hw]))
+    conv, pool, _, linear = sess.last_npu_profile().records
+    sess.close()
+    assert conv.kernel_ns > 0 and pool.duration_ns == 0, (conv, pool)
+    assert linear.duration_ns == linear.kernel_ns > 0, linear
