@@ -34,6 +34,7 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <stdexcept>
 
 #include "devmath.h"
@@ -47,6 +48,7 @@ constexpr int64_t kDirectBandBytes = 32 * 1024;  // LDS band of a workgroup at m
 struct DirectShape {
   int32_t C, H, W, O, OH, OW, k, stride, pad;
   int32_t blocks;  // 256-pixel blocks per image
+  int32_t total;   // of all images
   int32_t taps;
   int32_t BR, BW;         // rows per channel and row length of the LDS band
   uint32_t mBR, mBW, mOW;  // ceil(2^32 / d): exact quotients below 2^16
@@ -135,7 +137,9 @@ template <int MODE, int TAPS, int OB, bool BAND>
 __global__ __launch_bounds__(256) void conv_direct_kernel(const float* __restrict__ x, const float* __restrict__ wt,
                                                           const float* __restrict__ bias, float* __restrict__ y,
                                                           DirectShape s, int act, float act_param, int pool2) {
-  const int b = (int)blockIdx.x / s.blocks, blk = (int)blockIdx.x - b * s.blocks;
+  const int wg = (int)(blockIdx.z * gridDim.x + blockIdx.x);
+  if (wg >= s.total) return;
+  const int b = wg / s.blocks, blk = wg - b * s.blocks;
   const int o0 = (int)blockIdx.y * OB, o_n = s.O - o0;
   const int L = s.OH * s.OW, lane = (int)threadIdx.x & 63;
   const int pix_raw = blk * 256 + (int)threadIdx.x;
@@ -250,7 +254,7 @@ __global__ __launch_bounds__(256) void conv_direct_kernel(const float* __restric
 }
 
 bool conv_direct_supported(const ConvShape& cs) {
-  // 32-bit pixel and plane indexes, workgroups in grid.x
+  // 32-bit pixel, plane and workgroup indexes
   return cs.C * cs.k * cs.k <= kDirectConvTaps && cs.O <= 64 && cs.H * cs.W < (int64_t(1) << 29) &&
          cs.OH * cs.OW < (int64_t(1) << 29) && cs.n * ((cs.OH * cs.OW + 255) / 256) < (int64_t(1) << 31);
 }
@@ -266,7 +270,8 @@ static void launch_conv_direct_t(const float* x, const float* w, const float* bi
   if (L <= 0 || cs.n <= 0) return;
   DirectShape d{(int32_t)cs.C,      (int32_t)cs.H,   (int32_t)cs.W,              (int32_t)cs.O,
                       (int32_t)cs.OH,     (int32_t)cs.OW,  (int32_t)cs.k,              (int32_t)cs.stride,
-                      (int32_t)cs.pad,    (int32_t)((L + 255) / 256), (int32_t)(cs.C * cs.k * cs.k)};
+                      (int32_t)cs.pad,    (int32_t)((L + 255) / 256), 0,
+                      (int32_t)(cs.C * cs.k * cs.k)};
   // The band of a block: its output rows (one more where blocks start inside a
   // row) over the padded width.
   const int64_t rows = 256 % cs.OW == 0 ? 256 / cs.OW : (255 + cs.OW - 1) / cs.OW + 1;
@@ -282,7 +287,10 @@ static void launch_conv_direct_t(const float* x, const float* w, const float* bi
   // where that leaves fewer than 3 waves per SIMD.
   const int64_t wgs = cs.n * d.blocks;
   const int OB = band && cs.O > 16 && wgs * ((cs.O + 31) / 32) >= 768 ? 32 : 16;
-  const dim3 grid((unsigned)wgs, (unsigned)((cs.O + OB - 1) / OB));
+  d.total = (int32_t)wgs;
+  // a grid dimension holds fewer than 2^32 threads: the rest goes into z
+  constexpr int64_t kMaxX = int64_t(1) << 22;
+  const dim3 grid((unsigned)std::min(wgs, kMaxX), (unsigned)((cs.O + OB - 1) / OB), (unsigned)((wgs + kMaxX - 1) / kMaxX));
 #define RG_CD(T, B, BD)                                                                                            \
   RG_LAUNCH((conv_direct_kernel<MODE, T, B, BD>), grid, dim3(256), BD ? (unsigned)(cs.C * BR * BW * 4) : 0u, s, x, \
             w, bias, y, d, act, act_param, pool2)

@@ -348,8 +348,10 @@ static bool conv_mfma_tile(const ConvShape& cs, bool f16, bool pool, ConvMfmaTil
     const int64_t lds = std::max(band + TG * ob * 64, pool ? ob * (64 * pn + 4) * 4 : int64_t(0));
     const int64_t ty = (used + RB - 1) / RB, tx = (cs.OW + XB - 1) / XB, to = (cs.O + ob - 1) / ob;
     const int64_t grid = cs.n * ty * tx * to;
-    // quotients by multiplication are exact while dividend * divisor < 2^32
-    if (4 * BR * BC >= 65536 || BC >= 65536 || BR >= 65536 || lds > cmf::kMaxLds || grid >= (int64_t(1) << 31)) {
+    // quotients by multiplication are exact while dividend * divisor < 2^32; a grid
+    // holds fewer than 2^32 threads
+    if (4 * BR * BC >= 65536 || BC >= 65536 || BR >= 65536 || lds > cmf::kMaxLds ||
+        grid * cmf::kThreads >= (int64_t(1) << 32)) {
       pn = smaller;
       continue;
     }

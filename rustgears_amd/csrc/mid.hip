@@ -322,6 +322,12 @@ static int64_t mid_rounds(const MidTile& t, int64_t M, int64_t N) {
   return (((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn) + 255) / 256;
 }
 
+// A grid holds fewer than 2^32 threads (an operand's zero columns may take one
+// more column of tiles).
+static bool mid_grid_fits(const MidTile& t, int64_t M, int64_t N) {
+  return ((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn + 1) * mid::kThreads < (int64_t(1) << 32);
+}
+
 // The tile with the least estimated time: a CU's K blocks at 40 bytes a clock
 // of loads or one MFMA every 16 clocks per SIMD, whichever is more, over the
 // rounds of one workgroup per CU, plus 1 us a round and 2.5 us a launch.  FP32
@@ -333,29 +339,30 @@ static int64_t mid_rounds(const MidTile& t, int64_t M, int64_t N) {
 // rows) it and gemm_f32_us together took the fastest kernel or one within 1% on
 // average, 14% at most.
 int mid_choice(int mode, int64_t M, int64_t N, int64_t kb, double* us) {
-  int best = 0;
+  int best = -1;
   double best_us = 0.0;
   for (int i = 0; i < kMidTileCount; i++) {
     const MidTile& t = kMidTiles[i];
+    if (!mid_grid_fits(t, M, N)) continue;
     const double rounds = (double)mid_rounds(t, M, N), steps = (double)(kb / 64);
     const double load = steps * (t.tm + t.tn) * 64.0 / 40.0;
     const double mfma = steps * (t.tm / 16) * (t.tn / 16) * (mode == kModeF32 ? 128.0 : 16.0) / 4.0;
     const double work = mode == kModeF32 ? load + mfma + t.tm * t.tn : load > mfma ? load : mfma;
     const double c = 2.5 + rounds * (1.0 + work / 2400.0);
-    if (i == 0 || c < best_us) {
+    if (best < 0 || c < best_us) {
       best = i;
       best_us = c;
     }
   }
   if (us) *us = best_us;
-  return best;
+  return best < 0 ? 0 : best;
 }
 
 bool gemm_mid_supported(int64_t M, int64_t N, int64_t lda, int64_t kb) {
   // 32-bit offsets within a tile's rows, 32-bit sizes
   return M > 0 && N > 0 && M < (int64_t(1) << 31) - 256 && N < (int64_t(1) << 31) - 256 && kb > 0 && kb % 64 == 0 &&
          lda % 16 == 0 && 128 * lda < (int64_t(1) << 31) && 128 * kb < (int64_t(1) << 31) &&
-         ((M + 15) / 16) * ((N + 15) / 16) < (int64_t(1) << 31);
+         (mid_grid_fits({128, 64}, M, N) || mid_grid_fits({64, 128}, M, N));
 }
 
 template <int MODE, int FM, int FN, int KS, int STAGES>
