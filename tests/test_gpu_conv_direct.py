@@ -51,3 +51,18 @@ def test_fp32_infinite_inputs(rg, ref, c, k, hw, relu):
     for pool in (False, True) if oh % 2 == 0 and ow in (16, 32) else (False,):
         y = _run(rg, ref, c, 20, k, 1, pad, x, relu, pool)
     assert relu or np.isinf(y).any()
+
+
+@pytest.mark.parametrize("precision", ["f32", "f16"])
+@pytest.mark.parametrize("n,c,o,k,stride,pad,hw,relu,pool", [
+    # images too wide for the LDS band (32 KiB)
+    (2, 3, 20, 3, 1, 1, (6, 700), True, False), (2, 3, 64, 3, 2, 1, (7, 1500), False, False),
+    (1, 1, 17, 5, 1, 2, (5, 1400), True, False),
+    # 32 channels per thread (768 workgroups or more), the second block of them partly past the last channel
+    (400, 3, 40, 3, 1, 1, (16, 16), True, True), (400, 3, 60, 3, 1, 1, (16, 16), False, False),
+    (200, 3, 60, 3, 1, 1, (16, 32), True, True), (400, 2, 33, 3, 1, 1, (13, 19), False, False),
+    (800, 1, 64, 2, 1, 0, (9, 17), True, False),
+], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_wide_images_and_many_channels(rg, ref, precision, n, c, o, k, stride, pad, hw, relu, pool):
+    rg.manual_seed(n)
+    _run(rg, ref, c, o, k, stride, pad, rg.randn([n, c, *hw]), relu, pool, precision)
