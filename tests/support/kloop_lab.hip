@@ -13,9 +13,9 @@
 //                    rotated, no DMA)
 //   mfma32*          the three above with v_mfma_i32_32x32x32_i8 (16 MFMAs
 //                    per step, the same wave tile and fragment reads)
-//   production/4     gemm_core.h big_kloop, the 4-stage DMA ring of the
-//                    product's 256 x 256 GEMM, on random A [8192, 4096] and
-//                    B [4096, 4096]
+//   production/4     gemm_core.h alternating_kloop, the 4-stage DMA ring and
+//                    opposite phases of the product's 256 x 256 GEMM, on
+//                    random A [8192, 4096] and B [4096, 4096]
 //   production/3     the same with a 3-stage ring
 //   wide/lds         4 waves of 128 x 128 (one per SIMD, 256 accumulators):
 //                    16 fragment reads per step for 64 MFMAs, 2/3 of the
@@ -265,8 +265,8 @@ __global__ __launch_bounds__(512, 1) void ring_loop(const int8_t* __restrict__ A
   for (int t = blockIdx.x; t < kTiles; t += gridDim.x) {
     int tm, tn;
     tile_coords(t, 32, 16, tm, tn);
-    big_kloop<256, 256, 2, 4, STAGES, 8, kModeI8>(smem, A, B, 4096, (int64_t)tm * 256, (int64_t)tn * 256, 0, kSteps,
-                                                  wave, wm, wn, lane, acc);
+    alternating_kloop<8, STAGES, kModeI8>(smem, A, B, 4096, (int64_t)tm * 256, (int64_t)tn * 256, kSteps, wave, wm, wn,
+                                          lane, acc);
 #pragma unroll
     for (int i = 0; i < 8; i++)
 #pragma unroll
